@@ -212,10 +212,10 @@ int vdn_fp8_gemm(const void *xq, const float *x_scale, const void *wq, const flo
 /*
  * Bytes of workspace vdn_fp8_gemm_ws takes for an [M, N, K] GEMM on the current
  * device (0: the shape does not split). Only rows of K >= 8192 split: when the
- * 256 x 256 output tiles leave a last round of at most half the compute units,
- * those tiles run as several K slices whose binary32 partial sums go to the
- * workspace (256 KiB per slice), then a reduction kernel sums them, slice by
- * slice, and applies the epilogue.
+ * 256 x 256 output tiles leave a last round of at most half the compute units
+ * and no smaller tiles are faster, those tiles run as several K slices whose
+ * binary32 partial sums go to the workspace (256 KiB per slice), then a reduction
+ * kernel sums them, slice by slice, and applies the epilogue.
  * Replaces: nothing in the reference (torch._scaled_mm sizes its own workspace,
  *           src/models/ops/fp8_linear.py:272); the query for the next call.
  */
@@ -224,9 +224,9 @@ int vdn_fp8_gemm_workspace_size(int64_t M, int64_t N, int64_t K, int64_t *bytes)
 /*
  * vdn_fp8_gemm with a caller-provided split-K workspace (device memory, 16-byte
  * aligned, at least vdn_fp8_gemm_workspace_size bytes; NULL: no split, the same
- * call as vdn_fp8_gemm). The summation order of an output depends only on K,
- * its tile's position and the split, so a shape gives the same bits call after
- * call; a split shape's last-round tiles sum their K slices in binary32 after
+ * call as vdn_fp8_gemm). The summation order of an output depends only on K and
+ * the split, so a shape gives the same bits call after call, alone or as part of
+ * a larger one; a split shape's last-round tiles sum their K slices in binary32 after
  * the matrix cores, so their bits can differ from vdn_fp8_gemm's by a rounding.
  * Replaces: Fp8Linear.forward_quantized, src/models/ops/fp8_linear.py:270-277,
  *           as vdn_fp8_gemm does.

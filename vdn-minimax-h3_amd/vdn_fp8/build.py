@@ -32,8 +32,8 @@ LIB_PATH = os.path.join(_PKG, LIB_NAME)
 PROBE_SOURCES = ["stream_probe.hip", "mfma_probe.hip"]
 PROBE_PATH = os.path.join(_PKG, "libvdnprobe.so")
 
-SOURCES = ["capi.hip", "quantize.hip", "lora_requant.hip", "gemm.hip", "qk_prep.hip", "block_ops.hip"]
-HEADERS = ["vdn_common.h"]             # in csrc/
+SOURCES = ["capi.hip", "quantize.hip", "lora_requant.hip", "gemm.hip", "gemm_tile.hip", "qk_prep.hip", "block_ops.hip"]
+HEADERS = ["vdn_common.h", "gemm_common.h"]   # in csrc/
 PUBLIC_HEADERS = ["vdn_fp8.h"]         # in include/
 
 # -ffp-contract=off: the quantizers' binary32 arithmetic is bit-exact only as
@@ -90,7 +90,7 @@ def source_manifest(csrc=CSRC, include=INCLUDE, compiler=None):
 
 # The files that make each kernel family (its source plus the shared headers).
 KERNEL_FILES = {
-    "gemm": ["gemm.hip", "vdn_common.h", "vdn_fp8.h"],
+    "gemm": ["gemm.hip", "gemm_common.h", "vdn_common.h", "vdn_fp8.h"],
     "quantize": ["quantize.hip", "vdn_common.h", "vdn_fp8.h"],
     "lora_requant": ["lora_requant.hip", "quantize.hip", "vdn_common.h", "vdn_fp8.h"],
 }
