@@ -198,3 +198,23 @@ def test_merge_only_in_place(device):
     tol = _bf16_ulp(np.maximum(np.maximum(np.abs(w0), np.abs(wv - w0)), np.abs(wv)))
     assert np.all(np.abs(gv - wv) <= tol)
     assert np.mean(got != want) <= 2e-3
+
+
+@pytest.mark.parametrize("N,K,r", [(1, 5376, 8), (33, 5376, 64), (257, 5376, 32), (40, 5136, 64), (9, 5360, 16),
+                                   (5, 5392, 64)])
+@pytest.mark.parametrize("merged", [False, True])
+def test_requant_lora_21_chunks(device, N, K, r, merged):
+    """Rows of 5121 to 5376 elements, whose 21st chunk of 256 columns is a part of its own (K =
+    5392: past it, two passes). Codes and scales bit-exact with the oracle: the factors are
+    small integers over powers of two, so the update is exact in any order."""
+    print(f"lora requant, 21 chunks: N={N} K={K} r={r} merged={merged}", flush=True)
+    rng = np.random.default_rng(N + K + r)
+    w = O.bf16_encode(rng.standard_normal((N, K), dtype=np.float32) * 0.02)
+    a = O.bf16_encode((rng.integers(-3, 4, (r, K)) / 32.0).astype(np.float32))
+    b = O.bf16_encode((rng.integers(-3, 4, (N, r)) / 64.0).astype(np.float32))
+    gq, gs, gm = _requant(w, device, lora=(from_bits(a, device), from_bits(b, device), 0.5), merged=merged)
+    want = O.lora_merge(w, a, b, 0.5)
+    wq, ws = O.quantize_weight(want)
+    assert np.array_equal(gs.view(np.uint32), ws.view(np.uint32))
+    assert np.all(same_codes(gq, wq))
+    assert gm is None or np.array_equal(gm, want)

@@ -8,7 +8,7 @@
 // quantizes it in eager torch (fp8_linear.py:262-267): several full passes over
 // W plus the write-back of W'. Here W' is never stored unless asked for.
 //
-// Two kernels. k_lora_rows (further down; rank <= 64, K <= 5120, 16-byte rows)
+// Two kernels. k_lora_rows (further down; rank <= 64, K <= 5376, 16-byte rows)
 // reads W once: a workgroup holds a group of whole rows of W' in registers
 // until their maximum is known, then writes the codes. k_lora_stripes (first)
 // serves everything else -- ranks up to 128, longer rows, unaligned operands,
@@ -410,7 +410,7 @@ __global__ __launch_bounds__(kThreads) void k_lora_stripes(Args p)
 // columns advance in 256-wide chunks; wave w merges columns 32 w .. 32 w + 31 of
 // each chunk for all 32 rows, so a lane (row n = lane % 32, half h = lane / 32)
 // holds 16 consecutive columns of one row per chunk: all of its row's share of
-// W' stays in VGPRs (8 words a chunk, 160 at K = 5120) until the row maximum is
+// W' stays in VGPRs (8 words a chunk, 168 at K = 5376) until the row maximum is
 // known, and W is read from HBM exactly once.
 //
 // The rank-r update is v_mfma_f32_32x32x16_bf16 with MFMA row i = a column of
@@ -441,7 +441,7 @@ constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * kLanes;   // 512
 constexpr int kRows = 32;                   // rows of W per group (at most)
 constexpr int kChunk = 256;                 // columns per chunk (32 per wave)
-constexpr int kMaxChunks = 20;              // K <= 5120
+constexpr int kMaxChunks = 21;              // K <= 5376
 constexpr int kWStages = 4;                 // W chunks in LDS (16 KiB each)
 constexpr int kAStages = 3;                 // A slices in LDS (RP x 512 bytes each)
 constexpr int kRowB = kChunk * 2;           // bytes of one row of a chunk (W) or one rank row of a slice (A)
@@ -589,10 +589,11 @@ __global__ __launch_bounds__(rows::kThreads) void k_lora_rows(RowArgs p)
     constexpr int kRedOff = kWArea + kAArea - 1024;
     constexpr int kPartC = (2 * kRows * (4 * kChunk + 16) <= kAArea - 1024) ? 4
                            : (2 * kRows * (2 * kChunk + 16) <= kAArea - 1024) ? 2 : 1;
-    constexpr int kParts = NCH / kPartC;
+    constexpr int kParts = (NCH + kPartC - 1) / kPartC;
     constexpr int kCRow = kPartC * kChunk + 16;
     constexpr int kCBuf = kRows * kCRow;
-    static_assert(NCH % kPartC == 0 && 2 * kCBuf <= kAArea - 1024, "codes staging exceeds the A area");
+    // (the last part may hold fewer chunks: its missing columns lie past K and store nothing)
+    static_assert(2 * kCBuf <= kAArea - 1024, "codes staging exceeds the A area");
     // One 1 KiB store covers kRowsPerStore rows of a part; a wave stores kPartC of them
     // per part, one while each chunk of the next part is formed.
     constexpr int kRowsPerStore = 1024 / (kPartC * kChunk);
@@ -894,7 +895,7 @@ __global__ __launch_bounds__(rows::kThreads) void k_lora_rows(RowArgs p)
             uint8_t* const cst = smem + kWArea + (q % 2) * kCBuf;
 #pragma unroll
             for (int j = 0; j < kPartC; ++j) {
-                codes_chunk(q * kPartC + j, q * kPartC, cst);
+                if (q * kPartC + j < NCH) codes_chunk(q * kPartC + j, q * kPartC, cst);
                 if (q >= 1) store_piece((q - 1) * kPartC, j);
             }
             rows_sync<63>();
@@ -994,7 +995,10 @@ int launch_lora_requant(const uint16_t* w, int64_t N, int64_t K, int64_t ldw, co
     const int cus = device_cus();
     if (cus <= 0) return set_error(VDN_FP8_ELAUNCH, "requantize_weight: cannot query the device's compute units");
     // One pass with the rows in registers: codes wanted, rank <= 64 with 16-byte B
-    // rows, K <= 5120, 16-byte rows everywhere.
+    // rows, K <= 5376, 16-byte rows everywhere. (21 chunks are what the registers hold: 248 of
+    // 256 at rank <= 32, one spilled at rank 64, five with the merged rows written too. H3's
+    // 5376 columns against the two passes, W from HBM: [7168, 5376] rank 64 50.1 -> 27.6 us,
+    // [28672, 5376] 166 -> 108 us, rank 16 157 -> 90 us, with the merged weight 273 -> 178 us.)
     const bool one_pass = !merge_only && rank <= 64 && b_vec && K <= (int64_t)rows::kChunk * rows::kMaxChunks &&
                           aligned(w, 16) && ldw % 8 == 0 && aligned(wq, 16) && ldq % 16 == 0 &&
                           (!w_merged || aligned(w_merged, 16)) && (int64_t)rows::kRows * ldw * 2 <= 0x7fffffffLL &&
@@ -1008,7 +1012,7 @@ int launch_lora_requant(const uint16_t* w, int64_t N, int64_t K, int64_t ldw, co
         RowArgs r{w, N, K, ldw, a, b, rank, lora_scale, wq, ldq, w_scale, w_merged,
                   (int)((K + rows::kChunk - 1) / rows::kChunk), rows_pg, (int)((N + rows_pg - 1) / rows_pg)};
         const dim3 grid((unsigned)min((int64_t)r.groups, (int64_t)cus)), block(rows::kThreads);
-        // chunk-count instances: 8 (K <= 2048), 16 (K <= 4096), 20 (K <= 5120); chunks past
+        // chunk-count instances: 8 (K <= 2048), 16 (K <= 4096), 20 (K <= 5120), 21; chunks past
         // K read nothing and store nothing
 #define VDN_LORA_ROWS(R, C)                                                                            \
     do {                                                                                               \
@@ -1019,7 +1023,8 @@ int launch_lora_requant(const uint16_t* w, int64_t N, int64_t K, int64_t ldw, co
     do {                                                 \
         if (r.nch <= 8) VDN_LORA_ROWS(R, 8);             \
         else if (r.nch <= 16) VDN_LORA_ROWS(R, 16);      \
-        else VDN_LORA_ROWS(R, 20);                       \
+        else if (r.nch <= 20) VDN_LORA_ROWS(R, 20);           \
+        else VDN_LORA_ROWS(R, 21);                       \
     } while (0)
         if (rank <= 32) VDN_LORA_ROWS_RP(32);
         else VDN_LORA_ROWS_RP(64);
