@@ -240,6 +240,22 @@ int vdn_fp8_gemm_ws(const void *xq, const float *x_scale, const void *wq, const 
                     hipStream_t stream);
 
 /*
+ * vdn_fp8_gemm_ws with a binary16 or binary32 output (dtype VDN_FP8_DTYPE_F16 or _F32) and
+ * a bias of that type (or NULL), for models that do not run in bf16:
+ *   v         = T(x_scale[m] * w_scale[n] * acc[m][n])
+ *   out[m][n] = T(v + bias[n])
+ * rounded where the reference's sequence rounds: _scaled_mm with that out_dtype, then
+ * `out + bias`.
+ * Replaces: Fp8Linear.forward_quantized, src/models/ops/fp8_linear.py:270-277, with a
+ *           binary16 or binary32 out_dtype.
+ * Requires: as vdn_fp8_gemm_ws; a binary32 out 16-byte aligned.
+ */
+int vdn_fp8_gemm_typed(const void *xq, const float *x_scale, const void *wq, const float *w_scale,
+                       int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
+                       const void *bias, int dtype, void *out, int64_t ldo,
+                       void *workspace, int64_t workspace_bytes, hipStream_t stream);
+
+/*
  * vdn_fp8_gemm_ws without the workspace argument and without allocating: a split
  * shape uses a static 64 MiB device array of the library instead (one per GPU,
  * held until the process ends; its address is looked up on the first call on

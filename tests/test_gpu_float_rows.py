@@ -1,0 +1,86 @@
+"""GPU: float16 / float32 rows through the one-read quantizers and the GEMM's typed output.
+
+The quantizer's row widths cover each register count's edges and the two-sweep kernel past
+them; besides ordinary values every row holds elements at, one ulp below and one above each
+e4m3 rounding boundary times the row's scale, where a quotient off by one ulp would change
+the code. The GEMM's float16 / float32 output with its bias must give the bits of the binary32
+product followed by torch's own cast and add."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+import vdn_fp8
+import vdn_fp8._lib as L
+from conftest import codes, same_codes
+
+pytestmark = pytest.mark.gpu
+
+
+def _boundaries():
+    """The positive midpoints between neighbouring e4m3 values (and zero), in float64."""
+    c = torch.arange(0, 127, dtype=torch.uint8).view(torch.float8_e4m3fn).double().numpy()
+    return (c[1:] + c[:-1]) / 2
+
+
+def _row(rng, K, dtype, amax):
+    t = np.float32 if dtype == torch.float32 else np.float16
+    x = rng.standard_normal(K) * amax / 6
+    scale = np.float64(np.float32(np.float32(t(amax)) / np.float32(448.0)))
+    b = t(_boundaries() * scale)
+    near = np.concatenate([b, np.nextafter(b, t(np.inf)), np.nextafter(b, t(0))])[:max(0, K - 1)]
+    x = t(np.clip(x, -amax, amax))
+    at = rng.permutation(K - 1)[:near.size] + 1
+    x[at] = near * t(rng.choice([-1, 1]))
+    x[0] = t(amax)
+    return np.clip(x, -t(amax), t(amax))
+
+
+@pytest.mark.parametrize("weight", [False, True])
+@pytest.mark.parametrize("dtype,widths", [
+    (torch.float32, (8, 1016, 1024, 1032, 4096, 5120, 8192, 12296, 16384, 16392)),
+    (torch.float16, (8, 2040, 2048, 2056, 8192, 13824, 24576, 32768, 32776))])
+def test_float_rows_bit_exact(device, dtype, widths, weight):
+    rng = np.random.default_rng(5)
+    for K in widths:
+        print(f"float rows {dtype} K={K} weight={weight}", flush=True)
+        rows = [_row(rng, K, dtype, a) for a in (1.0, 3.7, 448.0, 1.5e-3, 6.1e4 if dtype == torch.float16 else 3e38)]
+        x = torch.from_numpy(np.stack(rows + [np.zeros_like(rows[0]), -rows[0]]))
+        if weight:
+            q, s = vdn_fp8.requantize_weight(x.to(device))
+            want_q, want_s = O.quantize_weight_float(x.numpy())
+        else:
+            q, s = vdn_fp8.quantize_rows(x.to(device))
+            want_q, want_s = O.quantize_rows_float(x.numpy())
+        assert same_codes(codes(q), want_q).all()
+        assert np.array_equal(s.cpu().numpy().reshape(-1).view(np.uint32), want_s.view(np.uint32))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("M,N,K", [(1, 4, 16), (77, 260, 400), (700, 1032, 2048), (4096, 4096, 512), (520, 1028, 8192)])
+def test_typed_output_is_the_cast_and_the_add(device, dtype, M, N, K):
+    """(4096, 4096: whole rounds of the persistent kernel; 520 x 1028 x 8192: split along K.)"""
+    print(f"typed gemm {dtype} [{M}, {N}, {K}]", flush=True)
+    g = torch.Generator(device=device).manual_seed(M + N + K)
+    lin = torch.nn.Linear(K, N, device=device, dtype=dtype)
+    with torch.no_grad():
+        lin.weight.copy_(0.02 * torch.randn(N, K, device=device, generator=g))
+        lin.bias.copy_(torch.randn(N, device=device, generator=g))
+    f = vdn_fp8.Fp8Linear(lin)
+    xq, xs = vdn_fp8.quantize_rows((3 * torch.randn(M, K, device=device, generator=g)).to(dtype))
+    xs[0] *= 1e9                       # float16 outputs that overflow
+    with torch.no_grad():
+        got = f.forward_quantized(xq, xs, out_dtype=dtype)
+    ws = torch.empty(max(16, vdn_fp8.fp8_linear.gemm_workspace_bytes(M, N, K, xq.device)), device=device, dtype=torch.uint8)
+    prod = torch.empty(M, N, device=device, dtype=torch.float32)
+    ptr = lambda t: t.data_ptr()
+    L.check(L.load().vdn_fp8_gemm_ws(ptr(xq), ptr(xs), ptr(f.weight_fp8), ptr(f.weight_scale), M, N, K, K, K, None,
+                                     L.EPI_F32, None, None, 0, 0, None, 0, ptr(prod), N, ptr(ws), ws.numel(),
+                                     torch.cuda.current_stream().cuda_stream), "gemm")
+    want = prod.to(dtype) + f.bias.detach()
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    # a bias that takes a gradient, or of another type, keeps the reference's own op
+    assert f.forward_quantized(xq, xs, out_dtype=dtype).requires_grad
+    f.bias = torch.nn.Parameter(f.bias.detach().double(), requires_grad=False)
+    assert f.forward_quantized(xq, xs, out_dtype=dtype).dtype == torch.float64

@@ -145,15 +145,15 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& p, const uint8_t* 
     constexpr int U = (XB + 1) / 2;             // 32-row bands of the wave (the last one 16 rows when XB is odd)
     const int wn = wave & 1, wm = wave >> 1;
     if constexpr (EPI == VDN_FP8_EPI_F32) {
-        // binary32 output x_scale * w_scale * acc, stored from the accumulators: 16 bytes
-        // (4 consecutive n of one m) per accumulator and lane; N % 4 == 0 keeps n .. n + 3
-        // inside a row whenever n is
+        // binary32 (or binary16) rows, stored from the accumulators: 4 consecutive n of one m
+        // per accumulator and lane; N % 4 == 0 keeps n .. n + 3 inside a row whenever n is
         uint32_t zero;
         asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
         const int el = (int)(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) + zero);
         const int fr = el & 15, fg = el >> 4;
         const float* s_sw = reinterpret_cast<const float*>(scal);
         const float* s_sx = reinterpret_cast<const float*>(scal + 1024);
+        const bool half = p.out_type == VDN_FP8_DTYPE_F16, has_bias = p.bias != nullptr;
         float* out = reinterpret_cast<float*>(p.out);
 #pragma unroll
         for (int j = 0; j < XB; ++j) {
@@ -166,10 +166,16 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& p, const uint8_t* 
                 const int nl = wn * 128 + 16 * i + 4 * fg;
                 const int64_t n = n0 + nl;
                 const float4 sw = *reinterpret_cast<const float4*>(s_sw + nl);
-                if (m < p.M && n < p.N)
-                    *reinterpret_cast<float4*>(out + m * p.ldo + n) =
-                        make_float4(acc[i][j][0] * (sxm * sw.x), acc[i][j][1] * (sxm * sw.y),
-                                    acc[i][j][2] * (sxm * sw.z), acc[i][j][3] * (sxm * sw.w));
+                const float v[4] = {acc[i][j][0] * (sxm * sw.x), acc[i][j][1] * (sxm * sw.y),
+                                    acc[i][j][2] * (sxm * sw.z), acc[i][j][3] * (sxm * sw.w)};
+                if (m < p.M && n < p.N) {
+                    if (half)
+                        *reinterpret_cast<uint2*>(p.out + m * p.ldo + n) =
+                            finish_f16x4(v, reinterpret_cast<const uint16_t*>(scal + 2048) + nl, has_bias);
+                    else
+                        *reinterpret_cast<float4*>(out + m * p.ldo + n) =
+                            finish_f32x4(v, reinterpret_cast<const float*>(scal + 2048) + nl, has_bias);
+                }
                 acc[i][j] = f32x4_t{};   // the next tile starts from zero
             }
         }
@@ -547,7 +553,10 @@ void k_gemm_fp8(GemmArgs p)
             const int64_t m0 = (int64_t)tm * TM, n0 = (int64_t)tn * BN;
             if (wave == 0) { base = p.sw + n0; bytes = min(p.N - n0, (int64_t)256) * 4; }
             else if (wave == 1) { base = p.sx + m0; bytes = min(p.M - m0, (int64_t)256) * 4; }
-            else if (wave == 2) { if (p.bias) { base = p.bias + n0; bytes = min(p.N - n0, (int64_t)512) * 2; } }
+            else if (wave == 2) {
+                const int64_t e = EPI == VDN_FP8_EPI_F32 && p.out_type == VDN_FP8_DTYPE_F32 ? 4 : 2;
+                if (p.bias) { base = reinterpret_cast<const uint8_t*>(p.bias) + n0 * e; bytes = min((p.N - n0) * e, (int64_t)1024); }
+            }
             else if (EPI == VDN_FP8_EPI_GATE && FAST) { base = p.gate + n0; bytes = min(p.N - n0, (int64_t)512) * 2; }
             else if (p.gate_index) { base = p.gate_index + m0; bytes = min(p.M - m0, (int64_t)256) * 4; }
         }
@@ -726,8 +735,9 @@ __device__ __forceinline__ void stage_tile_vectors(const GemmArgs& p, uint8_t* s
     const int64_t nn = min(p.N - n0, (int64_t)256), mm = min(p.M - m0, (int64_t)256);
     const __amdgpu_buffer_rsrc_t swr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.sw + n0), 0, (int)(nn * 4), kRsrcWord3);
     const __amdgpu_buffer_rsrc_t sxr = __builtin_amdgcn_make_buffer_rsrc((void*)(p.sx + m0), 0, (int)(mm * 4), kRsrcWord3);
+    const bool b32 = EPI == VDN_FP8_EPI_F32 && p.out_type == VDN_FP8_DTYPE_F32;   // a binary32 bias: 16 bytes per lane
     const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(p.bias ? p.bias + n0 : nullptr), 0, p.bias ? (int)(nn * 2) : 0, kRsrcWord3);
+        (void*)(p.bias ? p.bias + n0 * (b32 ? 2 : 1) : nullptr), 0, p.bias ? (int)(nn * (b32 ? 4 : 2)) : 0, kRsrcWord3);
     const bool grow = EPI == VDN_FP8_EPI_GATE && FAST;
     const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(
         grow ? (void*)(p.gate + n0) : (void*)(p.gate_index ? p.gate_index + m0 : nullptr), 0,
@@ -735,12 +745,14 @@ __device__ __forceinline__ void stage_tile_vectors(const GemmArgs& p, uint8_t* s
     const uint32_t l16 = (uint32_t)lane * 16, l8 = (uint32_t)lane * 8;
     const i32x4_t vsw = __builtin_amdgcn_raw_buffer_load_b128(swr, l16, 0, 0);
     const i32x4_t vsx = __builtin_amdgcn_raw_buffer_load_b128(sxr, l16, 0, 0);
-    const i32x2_t vb = __builtin_amdgcn_raw_buffer_load_b64(br, l8, 0, 0);
+    const i32x4_t vb4 = b32 ? __builtin_amdgcn_raw_buffer_load_b128(br, l16, 0, 0) : i32x4_t{};
+    const i32x2_t vb = b32 ? i32x2_t{} : __builtin_amdgcn_raw_buffer_load_b64(br, l8, 0, 0);
     const i32x4_t vg4 = grow ? i32x4_t{} : __builtin_amdgcn_raw_buffer_load_b128(gr, l16, 0, 0);
     const i32x2_t vg2 = grow ? __builtin_amdgcn_raw_buffer_load_b64(gr, l8, 0, 0) : i32x2_t{};
     *reinterpret_cast<i32x4_t*>(scal + l16) = vsw;
     *reinterpret_cast<i32x4_t*>(scal + 1024 + l16) = vsx;
-    *reinterpret_cast<i32x2_t*>(scal + 2048 + l8) = vb;
+    if (b32) *reinterpret_cast<i32x4_t*>(scal + 2048 + l16) = vb4;
+    else *reinterpret_cast<i32x2_t*>(scal + 2048 + l8) = vb;
     if (grow) *reinterpret_cast<i32x2_t*>(scal + 3072 + l8) = vg2;
     else *reinterpret_cast<i32x4_t*>(scal + 3072 + l16) = vg4;
 }
@@ -919,11 +931,12 @@ int gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t* bytes)
     return VDN_FP8_OK;
 }
 
-// The GEMM with an optional split-K workspace (ws NULL: no split).
+// The GEMM with an optional split-K workspace (ws NULL: no split). out_type: VDN_FP8_DTYPE_F16
+// or _F32 with VDN_FP8_EPI_F32 (bias of that type); -1: what the epilogue implies.
 int gemm_launch(const void* xq, const float* x_scale, const void* wq, const float* w_scale, int64_t M, int64_t N,
                 int64_t K, int64_t ldx, int64_t ldw, const void* bias, int epilogue, const void* gate,
                 const int32_t* gate_index, int64_t gate_rows, int64_t ldgate, const void* residual, int64_t ldres,
-                void* out, int64_t ldo, float* ws, int64_t ws_bytes, hipStream_t stream)
+                void* out, int64_t ldo, float* ws, int64_t ws_bytes, hipStream_t stream, int out_type)
 {
     if (M < 0 || N < 0 || K < 0) return set_error(VDN_FP8_EINVAL, "gemm: negative shape");
     if (M == 0 || N == 0) return VDN_FP8_OK;
@@ -943,9 +956,9 @@ int gemm_launch(const void* xq, const float* x_scale, const void* wq, const floa
         if (residual && (ldres < N || ldres % 4 || !aligned(residual, 8)))
             return set_error(VDN_FP8_EINVAL, "gemm: residual rows must be >= N and 8-byte aligned");
     } else if (epilogue == VDN_FP8_EPI_F32) {
-        if (bias || gate || residual || gate_index)
+        if ((bias && out_type < 0) || gate || residual || gate_index)
             return set_error(VDN_FP8_EINVAL, "gemm: the binary32 output takes no bias, gate or residual");
-        if (!aligned(out, 16)) return set_error(VDN_FP8_EINVAL, "gemm: the binary32 output must be 16-byte aligned");
+        if (out_type != VDN_FP8_DTYPE_F16 && !aligned(out, 16)) return set_error(VDN_FP8_EINVAL, "gemm: the binary32 output must be 16-byte aligned");
     } else if (epilogue != VDN_FP8_EPI_NONE && epilogue != VDN_FP8_EPI_GELU_TANH) {
         return set_error(VDN_FP8_EINVAL, "gemm: unknown epilogue %d", epilogue);
     }
@@ -971,7 +984,8 @@ int gemm_launch(const void* xq, const float* x_scale, const void* wq, const floa
     const GemmPlan plan = plan_gemm(M, N, K, cus, ws != nullptr, fast);
     GemmArgs p{(const uint8_t*)xq, x_scale, (const uint8_t*)wq, w_scale, M, N, K, ldx, ldw,
                (const uint16_t*)bias, (const uint16_t*)gate, gate_index, gate_rows, ldgate,
-               (const uint16_t*)residual, ldres, (uint16_t*)out, ldo, (int)tiles_m, (int)tiles_n,
+               (const uint16_t*)residual, ldres, (uint16_t*)out, ldo,
+               epilogue == VDN_FP8_EPI_F32 && out_type < 0 ? VDN_FP8_DTYPE_F32 : std::max(out_type, 0), (int)tiles_m, (int)tiles_n,
                kGroupM, plan.t_main, plan.splits, plan.units, ws};
     const bool tile_fast = out16 && (!gated || rows31);
     if (!plan.main) return launch_gemm_tile(p, plan.a, plan.b, 0, epilogue, tile_fast, stream);
@@ -1003,7 +1017,7 @@ int gemm_launch(const void* xq, const float* x_scale, const void* wq, const floa
     if (rows16 && !rows31 && !gate_broadcast) {
         // rows whose offsets pass 31 bits: the GEMM writing v, then the gated residual kernel
         const int st = gemm_launch(xq, x_scale, wq, w_scale, M, N, K, ldx, ldw, bias, VDN_FP8_EPI_NONE, nullptr, nullptr,
-                                   0, 0, nullptr, 0, out, ldo, ws, ws_bytes, stream);
+                                   0, 0, nullptr, 0, out, ldo, ws, ws_bytes, stream, -1);
         if (st != VDN_FP8_OK) return st;
         return launch_gated_residual((const uint16_t*)residual, ldres, (const uint16_t*)gate, ldgate, gate_index,
                                      gate_rows, (const uint16_t*)out, ldo, (uint16_t*)out, ldo, M, N, stream);
@@ -1036,7 +1050,7 @@ extern "C" int vdn_fp8_gemm(const void* xq, const float* x_scale, const void* wq
                             const void* residual, int64_t ldres, void* out, int64_t ldo, hipStream_t stream)
 {
     return gemm_launch(xq, x_scale, wq, w_scale, M, N, K, ldx, ldw, bias, epilogue, gate, gate_index, gate_rows,
-                       ldgate, residual, ldres, out, ldo, nullptr, 0, stream);
+                       ldgate, residual, ldres, out, ldo, nullptr, 0, stream, -1);
 }
 
 extern "C" int vdn_fp8_gemm_workspace_size(int64_t M, int64_t N, int64_t K, int64_t* bytes)
@@ -1052,7 +1066,17 @@ extern "C" int vdn_fp8_gemm_ws(const void* xq, const float* x_scale, const void*
                                int64_t workspace_bytes, hipStream_t stream)
 {
     return gemm_launch(xq, x_scale, wq, w_scale, M, N, K, ldx, ldw, bias, epilogue, gate, gate_index, gate_rows,
-                       ldgate, residual, ldres, out, ldo, (float*)workspace, workspace_bytes, stream);
+                       ldgate, residual, ldres, out, ldo, (float*)workspace, workspace_bytes, stream, -1);
+}
+
+extern "C" int vdn_fp8_gemm_typed(const void* xq, const float* x_scale, const void* wq, const float* w_scale, int64_t M,
+                                  int64_t N, int64_t K, int64_t ldx, int64_t ldw, const void* bias, int dtype, void* out,
+                                  int64_t ldo, void* workspace, int64_t workspace_bytes, hipStream_t stream)
+{
+    if (dtype != VDN_FP8_DTYPE_F16 && dtype != VDN_FP8_DTYPE_F32)
+        return set_error(VDN_FP8_EINVAL, "gemm_typed: the output is binary16 or binary32 (dtype %d)", dtype);
+    return gemm_launch(xq, x_scale, wq, w_scale, M, N, K, ldx, ldw, bias, VDN_FP8_EPI_F32, nullptr, nullptr, 0, 0, nullptr,
+                       0, out, ldo, (float*)workspace, workspace_bytes, stream, dtype);
 }
 
 // ---------------------------------------------------------------------------
@@ -1105,5 +1129,5 @@ extern "C" int vdn_fp8_gemm_noalloc(const void* xq, const float* x_scale, const 
         if (!ws) return set_error(VDN_FP8_ELAUNCH, "gemm_noalloc: cannot look up the scratch array on device %d", dev);
     }
     return gemm_launch(xq, x_scale, wq, w_scale, M, N, K, ldx, ldw, bias, epilogue, gate, gate_index, gate_rows,
-                       ldgate, residual, ldres, out, ldo, ws, ws ? kScratchBytes : 0, stream);
+                       ldgate, residual, ldres, out, ldo, ws, ws ? kScratchBytes : 0, stream, -1);
 }

@@ -23,7 +23,7 @@ struct GemmArgs {
     const uint8_t* wq;
     const float* sw;
     int64_t M, N, K, ldx, ldw;
-    const uint16_t* bias;
+    const uint16_t* bias;   // of the output's type (out_type)
     const uint16_t* gate;
     const int32_t* gate_index;
     int64_t gate_rows, ldgate;
@@ -31,6 +31,7 @@ struct GemmArgs {
     int64_t ldres;
     uint16_t* out;
     int64_t ldo;
+    int out_type;           // VDN_FP8_DTYPE_*: binary16 and binary32 with VDN_FP8_EPI_F32
     int tiles_m, tiles_n;
     int group_m;   // m-tiles per group of the tile order
     // Split of the last partial round along K (long rows only): the first t_main tiles
@@ -53,6 +54,31 @@ const GemmTile* gemm_tiles(int* count);
 // The tile kernel over the whole output (rest = 0), or over the last `rest` 256 x 256 tiles
 // from p.t_main on (a and b 4 or 8). epilogue: the C ABI's; fast: 16-byte rows throughout.
 int launch_gemm_tile(GemmArgs p, int a, int b, int rest, int epilogue, bool fast, hipStream_t stream);
+
+// Four outputs of a binary16 or binary32 row (VDN_FP8_EPI_F32): the binary32 product in the
+// output's type, then the bias of that type, rounded where the reference's cast and `out +
+// bias` round. b: the four bias values in LDS.
+__device__ __forceinline__ uint2 finish_f16x4(const float (&v)[4], const uint16_t* b, bool has_bias)
+{
+    _Float16 h[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float t = v[e];
+        asm volatile("" : "+v"(t));   // rounded to binary32 first (else one instruction multiplies and rounds to binary16)
+        h[e] = (_Float16)t;
+        if (has_bias) h[e] = (_Float16)((float)h[e] + (float)__builtin_bit_cast(_Float16, b[e]));
+    }
+    auto pair = [](_Float16 lo, _Float16 hi) {
+        return (uint32_t)__builtin_bit_cast(uint16_t, lo) | ((uint32_t)__builtin_bit_cast(uint16_t, hi) << 16);
+    };
+    return make_uint2(pair(h[0], h[1]), pair(h[2], h[3]));
+}
+
+__device__ __forceinline__ float4 finish_f32x4(const float (&v)[4], const float* b, bool has_bias)
+{
+    if (!has_bias) return make_float4(v[0], v[1], v[2], v[3]);
+    return make_float4(v[0] + b[0], v[1] + b[1], v[2] + b[2], v[3] + b[3]);
+}
 
 // Renumbers workgroup b so that XCD (b % 8) gets a contiguous run of tiles,
 // then maps the run index to (tile_m, tile_n) in groups of gm m-tiles.

@@ -63,7 +63,10 @@ void k_gemm_tile(GemmArgs p, int epi, int fast)
         int64_t bytes = 0;
         if (wave == 0) { base = p.sw + n0; bytes = min(p.N - n0, (int64_t)256) * 4; }
         else if (wave == 1) { base = p.sx + m0; bytes = min(p.M - m0, (int64_t)256) * 4; }
-        else if (wave == 2) { if (p.bias) { base = p.bias + n0; bytes = min(p.N - n0, (int64_t)512) * 2; } }
+        else if (wave == 2) {
+            const int64_t e = p.out_type == VDN_FP8_DTYPE_F32 ? 4 : 2;   // bytes of a bias value
+            if (p.bias) { base = reinterpret_cast<const uint8_t*>(p.bias) + n0 * e; bytes = min((p.N - n0) * e, (int64_t)1024); }
+        }
         else if (p.gate_index) { base = p.gate_index + m0; bytes = min(p.M - m0, (int64_t)256) * 4; }
         const i32x4_t r = rsrc_words(base, bytes);
         asm volatile("s_nop 4");   // SGPR write by VALU -> use as a buffer descriptor
@@ -161,8 +164,10 @@ void k_gemm_tile(GemmArgs p, int epi, int fast)
     const float* s_sx = reinterpret_cast<const float*>(smem + kScal + 1024);
     const uint16_t* s_bias = reinterpret_cast<const uint16_t*>(smem + kScal + 2048);
     const int32_t* s_gi = reinterpret_cast<const int32_t*>(smem + kScal + 3072);
-    if (epi == VDN_FP8_EPI_F32) {   // binary32 x_scale * w_scale * acc, from the accumulators
+    const bool has_bias = p.bias != nullptr;
+    if (epi == VDN_FP8_EPI_F32 && p.out_type == VDN_FP8_DTYPE_F32) {   // binary32 rows, from the accumulators
         float* out = reinterpret_cast<float*>(p.out);
+        const float* s_bf = reinterpret_cast<const float*>(smem + kScal + 2048);
 #pragma unroll
         for (int j = 0; j < B; ++j) {
             const int ml = 16 * (B * wm + j) + fr;
@@ -171,10 +176,10 @@ void k_gemm_tile(GemmArgs p, int epi, int fast)
             for (int i = 0; i < A; ++i) {
                 const int nl = 16 * (A * wn + i) + 4 * fg;
                 const float4 sw = *reinterpret_cast<const float4*>(s_sw + nl);
+                const float v[4] = {acc[i][j][0] * (sxm * sw.x), acc[i][j][1] * (sxm * sw.y),
+                                    acc[i][j][2] * (sxm * sw.z), acc[i][j][3] * (sxm * sw.w)};
                 if (m0 + ml < p.M && n0 + nl < p.N)
-                    *reinterpret_cast<float4*>(out + (m0 + ml) * p.ldo + n0 + nl) =
-                        make_float4(acc[i][j][0] * (sxm * sw.x), acc[i][j][1] * (sxm * sw.y), acc[i][j][2] * (sxm * sw.z),
-                                    acc[i][j][3] * (sxm * sw.w));
+                    *reinterpret_cast<float4*>(out + (m0 + ml) * p.ldo + n0 + nl) = finish_f32x4(v, s_bf + nl, has_bias);
             }
         }
         return;
@@ -182,18 +187,23 @@ void k_gemm_tile(GemmArgs p, int epi, int fast)
     uint8_t* const stg = smem + wave * 16 * B * RS;
     // the wave's 16 B x 16 A outputs, rounded where the reference rounds (a missing bias adds
     // -0, which leaves every value as it is), into its own staging rows
-    auto finish = [&](auto gelu) {
+    auto finish = [&](auto gelu, auto half) {
 #pragma unroll
         for (int i = 0; i < A; ++i) {
             const int nl = 16 * (A * wn + i) + 4 * fg;
             const float4 sw = *reinterpret_cast<const float4*>(s_sw + nl);
             const uint2 b = *reinterpret_cast<const uint2*>(s_bias + nl);
-            const bool hb = p.bias != nullptr;
-            const float b0 = hb ? bf16_lo(b.x) : -0.0f, b1 = hb ? bf16_hi(b.x) : -0.0f;
-            const float b2 = hb ? bf16_lo(b.y) : -0.0f, b3 = hb ? bf16_hi(b.y) : -0.0f;
+            const float b0 = has_bias ? bf16_lo(b.x) : -0.0f, b1 = has_bias ? bf16_hi(b.x) : -0.0f;
+            const float b2 = has_bias ? bf16_lo(b.y) : -0.0f, b3 = has_bias ? bf16_hi(b.y) : -0.0f;
 #pragma unroll
             for (int j = 0; j < B; ++j) {
                 const float sxm = s_sx[16 * (B * wm + j) + fr];
+                if (decltype(half)::value) {
+                    const float v[4] = {acc[i][j][0] * (sxm * sw.x), acc[i][j][1] * (sxm * sw.y),
+                                        acc[i][j][2] * (sxm * sw.z), acc[i][j][3] * (sxm * sw.w)};
+                    *reinterpret_cast<uint2*>(stg + (16 * j + fr) * RS + 32 * i + 8 * fg) = finish_f16x4(v, s_bias + nl, has_bias);
+                    continue;
+                }
                 uint32_t r01 = pack_bf16x2(acc[i][j][0] * (sxm * sw.x), acc[i][j][1] * (sxm * sw.y));
                 uint32_t r23 = pack_bf16x2(acc[i][j][2] * (sxm * sw.z), acc[i][j][3] * (sxm * sw.w));
                 asm volatile("" : "+v"(r01), "+v"(r23));   // each pair in one conversion
@@ -208,8 +218,9 @@ void k_gemm_tile(GemmArgs p, int epi, int fast)
             }
         }
     };
-    if (epi == VDN_FP8_EPI_GELU_TANH) finish(std::true_type{});
-    else finish(std::false_type{});
+    if (epi == VDN_FP8_EPI_GELU_TANH) finish(std::true_type{}, std::false_type{});
+    else if (epi == VDN_FP8_EPI_F32) finish(std::false_type{}, std::true_type{});   // binary16 rows
+    else finish(std::false_type{}, std::false_type{});
     // out = bf16(residual + gate[i] * v) on packed pairs, in the rows' layout
     const bool gated = epi == VDN_FP8_EPI_GATE, has_res = p.residual != nullptr;
     auto gate_pair = [&](uint32_t v, uint32_t g, uint32_t r) {

@@ -268,9 +268,10 @@ __global__ __launch_bounds__(kWavesPerBlock * kLanes) void k_swiglu_quant(
 // ---------------------------------------------------------------------------
 // binary32 and binary16 rows (the reference's quantizers load any float type
 // and compute in binary32, fp8_linear.py:72,77,89-90; its weight branch
-// divides in the weight's own type, fp8_linear.py:264-265). A path for
-// models that do not run in bf16: one wave per row and two sweeps (the row
-// maximum, then the codes, the second reading the row again), IEEE division.
+// divides in the weight's own type, fp8_linear.py:264-265), for models that
+// do not run in bf16. Quantizers: four waves per row, the row held in registers
+// (k_rowquant_float); rows past that, and SwiGLU, one wave per row and two sweeps
+// (the row maximum, then the codes, the second reading the row again).
 // ---------------------------------------------------------------------------
 
 // torch's cast to e4m3fn does not saturate: a magnitude above 464 (halfway
@@ -323,11 +324,92 @@ __device__ __forceinline__ void store_float_codes(uint8_t* yr, int64_t c, const 
                                                             pack_e4m3x4(q[4], q[5], q[6], q[7]));
 }
 
+// x / s correctly rounded, from r = RN(1 / s), for finite s >= 1e-12: two of Markstein's
+// corrections (div_by_scale has one, which suffices for the bf16 rows it was checked on
+// exhaustively). The first leaves a quotient within an ulp, from which the second rounds
+// correctly (P. Markstein, IBM J. Res. Dev. 34(1), 1990); where an operation of it could
+// underflow, the quotient is below e4m3's smallest half step and its code a signed zero.
+__device__ __forceinline__ float div_correct(float x, float s, float r)
+{
+    const float q = div_by_scale(x, s, r);
+    return __builtin_fmaf(-__builtin_fmaf(q, s, -x), r, q);
+}
+
+// Magnitude bits of 16 bytes of a row: their maximum orders as the magnitudes do, NaN above inf
+// (binary16 pairs as packed 16-bit maxima).
+template <typename T>
+__device__ __forceinline__ uint32_t float_absmax(uint32_t acc, uint4 v)
+{
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (sizeof(T) == 4) acc = max(acc, w[e] & 0x7fffffffu);
+        else acc = absmax_bf16x2(acc, w[e]);   // (sign bits off, packed 16-bit maximum: any 16-bit float)
+    }
+    return acc;
+}
+
+// One row per workgroup of four waves, 256 x CPL 16-byte pieces of it in registers between the
+// maximum and the cast: the row is read once and the quotients of a finite scale take five
+// operations instead of an IEEE division's dozen. Bound: HBM (6 or 3 bytes per element).
+// Against the two sweeps, one MI355X: [32760, 5120] binary32 240 -> 130 us (6.2 TB/s), binary16
+// 135 -> 77 us, [4096, 8192] binary32 45 -> 28 us.
+template <typename T, bool kWeight, int CPL>
+__global__ __launch_bounds__(kWavesPerBlock * kLanes) void k_rowquant_float(
+    const T* __restrict__ x, int64_t K, int64_t ldx, uint8_t* __restrict__ y, int64_t ldy, float* __restrict__ scale_out)
+{
+    using R = FloatRow<T>;
+    constexpr int kThreads = kWavesPerBlock * kLanes;
+    __shared__ uint32_t smax[kWavesPerBlock];
+    const int64_t row = blockIdx.x;
+    const int nch = (int)(K / R::kPer), tid = (int)threadIdx.x;
+    const uint4* xr = reinterpret_cast<const uint4*>(x + row * ldx);
+    uint4 v[CPL];
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) v[c] = tid + kThreads * c < nch ? load_once(xr + tid + kThreads * c) : make_uint4(0u, 0u, 0u, 0u);
+    uint32_t m = 0;
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) m = float_absmax<T>(m, v[c]);
+    if (sizeof(T) == 2) m = max(m & 0xffffu, m >> 16);
+    m = wave_max_u32(m);
+    if ((tid & (kLanes - 1)) == 0) smax[tid / kLanes] = m;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kWavesPerBlock; ++w) m = max(m, smax[w]);
+    const float amax = sizeof(T) == 4 ? __uint_as_float(m) : (float)__builtin_bit_cast(_Float16, (uint16_t)m);
+    const float scale = row_scale(__builtin_isnan(amax) ? __uint_as_float(0x7fc00000u) : amax);
+    if (tid == 0) scale_out[row] = scale;
+    const float sdiv = kWeight ? R::round(scale) : scale;
+    const float r = 1.0f / sdiv;
+    // (a binary16 weight's scale may round to zero or far below itself: IEEE division there)
+    constexpr bool kAlwaysIeee = kWeight && sizeof(T) == 2;
+    uint8_t* yr = y + row * ldy;
+    auto cast = [&](auto ieee) {
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) {
+            if (tid + kThreads * c >= nch) continue;
+            float f[8], q[8];
+            R::unpack(v[c], f);
+#pragma unroll
+            for (int e = 0; e < R::kPer; ++e) {
+                if (!decltype(ieee)::value) q[e] = div_correct(f[e], sdiv, r);
+                else {
+                    const float t = f[e] / sdiv;
+                    q[e] = e4m3_domain(kWeight ? R::round(t) : t);
+                }
+            }
+            store_float_codes<R::kPer>(yr, tid + kThreads * c, q);
+        }
+    };
+    if (!kAlwaysIeee && __builtin_isfinite(sdiv)) cast(std::false_type{});
+    else cast(std::true_type{});
+}
+
 //   scale[m] = max(max_k |x[m][k]| / 448, 1e-12)
 //   y[m][k]  = e4m3(x[m][k] / scale[m])                    (activations)
 //   y[m][k]  = e4m3(T(x[m][k] / T(scale[m])))              (kWeight: the weight's own type)
 template <typename T, bool kWeight>
-__global__ __launch_bounds__(kWavesPerBlock * kLanes) void k_rowquant_float(
+__global__ __launch_bounds__(kWavesPerBlock * kLanes) void k_rowquant_float_wide(
     const T* __restrict__ x, int64_t M, int64_t K, int64_t ldx,
     uint8_t* __restrict__ y, int64_t ldy, float* __restrict__ scale_out)
 {
@@ -1223,6 +1305,28 @@ int check_typed_rows(const char* what, const void* x, int dtype, int64_t M, int6
         return set_error(VDN_FP8_EINVAL, "%s: x must be 16-byte and y 8-byte aligned", what);
     return -1;   // go on
 }
+
+// The float row quantizers by the row's 16-byte pieces: 256 per workgroup and step, up to 16
+// steps in registers, past that the two sweeps.
+template <typename T, bool kWeight>
+int launch_rowquant_float(const char* what, const T* x, int64_t M, int64_t K, int64_t ldx, uint8_t* y, int64_t ldy,
+                          float* scale, hipStream_t stream)
+{
+    const dim3 block(kWavesPerBlock * kLanes);
+    const int64_t per = (K / FloatRow<T>::kPer + kWavesPerBlock * kLanes - 1) / (kWavesPerBlock * kLanes);
+    if (per > 16 || M > 0x7fffffff) {
+        const dim3 grid((unsigned)((M + kWavesPerBlock - 1) / kWavesPerBlock));
+        hipLaunchKernelGGL((k_rowquant_float_wide<T, kWeight>), grid, block, 0, stream, x, M, K, ldx, y, ldy, scale);
+        return check_launch(what);
+    }
+#define VDN_CASE(n)                                                                                            \
+    else if (per <= n)                                                                                         \
+        hipLaunchKernelGGL((k_rowquant_float<T, kWeight, n>), dim3((unsigned)M), block, 0, stream, x, K, ldx, y, ldy, scale);
+    if (false) {}
+    VDN_CASE(1) VDN_CASE(2) VDN_CASE(3) VDN_CASE(4) VDN_CASE(5) VDN_CASE(6) VDN_CASE(8) VDN_CASE(12) VDN_CASE(16)
+#undef VDN_CASE
+    return check_launch(what);
+}
 }  // namespace
 
 extern "C" int vdn_fp8_quantize_rows_typed(const void* x, int dtype, int64_t M, int64_t K, int64_t ldx, void* y,
@@ -1231,14 +1335,10 @@ extern "C" int vdn_fp8_quantize_rows_typed(const void* x, int dtype, int64_t M, 
     if (dtype == VDN_FP8_DTYPE_BF16) return vdn_fp8_quantize_rows(x, M, K, ldx, y, ldy, scale, stream);
     const int st = check_typed_rows("quantize_rows", x, dtype, M, K, ldx, K, y, ldy, scale);
     if (st >= 0) return st;
-    const dim3 grid((unsigned)((M + kWavesPerBlock - 1) / kWavesPerBlock)), block(kWavesPerBlock * kLanes);
     if (dtype == VDN_FP8_DTYPE_F32)
-        hipLaunchKernelGGL((k_rowquant_float<float, false>), grid, block, 0, stream, (const float*)x, M, K, ldx,
-                           (uint8_t*)y, ldy, scale);
-    else
-        hipLaunchKernelGGL((k_rowquant_float<_Float16, false>), grid, block, 0, stream, (const _Float16*)x, M, K,
-                           ldx, (uint8_t*)y, ldy, scale);
-    return check_launch("quantize_rows");
+        return launch_rowquant_float<float, false>("quantize_rows", (const float*)x, M, K, ldx, (uint8_t*)y, ldy, scale, stream);
+    return launch_rowquant_float<_Float16, false>("quantize_rows", (const _Float16*)x, M, K, ldx, (uint8_t*)y, ldy, scale,
+                                                  stream);
 }
 
 extern "C" int vdn_fp8_swiglu_quantize_rows_typed(const void* h, int dtype, int64_t M, int64_t K, int64_t ldh,
@@ -1264,12 +1364,9 @@ extern "C" int vdn_fp8_requantize_weight_typed(const void* w, int dtype, int64_t
         return vdn_fp8_requantize_weight(w, N, K, ldw, nullptr, nullptr, 0, 0.0f, wq, ldq, w_scale, nullptr, stream);
     const int st = check_typed_rows("requantize_weight", w, dtype, N, K, ldw, K, wq, ldq, w_scale);
     if (st >= 0) return st;
-    const dim3 grid((unsigned)((N + kWavesPerBlock - 1) / kWavesPerBlock)), block(kWavesPerBlock * kLanes);
     if (dtype == VDN_FP8_DTYPE_F32)
-        hipLaunchKernelGGL((k_rowquant_float<float, true>), grid, block, 0, stream, (const float*)w, N, K, ldw,
-                           (uint8_t*)wq, ldq, w_scale);
-    else
-        hipLaunchKernelGGL((k_rowquant_float<_Float16, true>), grid, block, 0, stream, (const _Float16*)w, N, K, ldw,
-                           (uint8_t*)wq, ldq, w_scale);
-    return check_launch("requantize_weight");
+        return launch_rowquant_float<float, true>("requantize_weight", (const float*)w, N, K, ldw, (uint8_t*)wq, ldq, w_scale,
+                                                  stream);
+    return launch_rowquant_float<_Float16, true>("requantize_weight", (const _Float16*)w, N, K, ldw, (uint8_t*)wq, ldq, w_scale,
+                                                 stream);
 }

@@ -394,19 +394,21 @@ class Fp8Linear(nn.Module):
         ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8) if ws_bytes else None
         if out_dtype != torch.bfloat16:
             # the reference's _scaled_mm with a float16 / float32 out_dtype, then `out + bias`
-            # (fp8_linear.py:272-276): the GEMM writes the binary32 product, and the
-            # rounding to float16 and the bias add are the reference's own two ops
-            out = torch.empty(M, N, device=dev, dtype=torch.float32)
-            _lib.check(lib.vdn_fp8_gemm_ws(_ptr(x_fp8), _ptr(x_scale), _ptr(self.weight_fp8),
-                                           _ptr(self.weight_scale), M, N, K, x_fp8.stride(0), K,
-                                           None, _lib.EPI_F32, None, None, 0, 0, None, 0,
-                                           _ptr(out), N, _ptr(ws), ws_bytes, _stream(x_fp8)),
+            # (fp8_linear.py:272-276), with the cast and a bias Parameter of that type in the
+            # GEMM's epilogue ([1111, 4100, 4112] float16: two passes over the output and
+            # their launches less). Any other bias (one whose type promotes, that takes a
+            # gradient, or that is no plain Parameter) is added as the reference's own op.
+            bias = self.bias
+            fused = (type(bias) is nn.Parameter and bias.dtype == out_dtype and bias.shape == (N,)
+                     and bias.device == dev and not (torch.is_grad_enabled() and bias.requires_grad))
+            b = _aligned16(bias.detach().contiguous()) if fused else None
+            out = torch.empty(M, N, device=dev, dtype=out_dtype)
+            _lib.check(lib.vdn_fp8_gemm_typed(_ptr(x_fp8), _ptr(x_scale), _ptr(self.weight_fp8),
+                                              _ptr(self.weight_scale), M, N, K, x_fp8.stride(0), K,
+                                              _ptr(b), _DTYPES[out_dtype], _ptr(out), N, _ptr(ws), ws_bytes,
+                                              _stream(x_fp8)),
                        "fp8 gemm")
-            if out_dtype != torch.float32:
-                out = out.to(out_dtype)
-            if self.bias is not None:
-                out = out + self.bias
-            return out
+            return out if bias is None or fused else out + bias
         out = torch.empty(M, N, device=dev, dtype=torch.bfloat16)
         epi = _EPILOGUES.get(epilogue)
         if epi is None:
