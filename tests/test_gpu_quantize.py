@@ -150,6 +150,31 @@ def test_swiglu_quantize(device, M, K):
     assert np.all((diff <= 1) | (np.abs(gv - wv) <= 0.07 * np.abs(wv) + 1e-30)), "a code is off by more than one step"
 
 
+@pytest.mark.parametrize("K", [8192, 8200, 12288, 12296, 14328, 14336, 14344, 16384])
+def test_swiglu_quantize_split_rows(device, K):
+    """Four waves per row at the chunk counts' edges, rows of a wider tensor: the columns past
+    2K hold NaN, which a read past either half would carry into the row's scale, and the codes'
+    padding stays as it was. The codes and scales are those of the rows alone (same kernel, same
+    chunks: bit for bit), and of the oracle within test_swiglu_quantize's bounds."""
+    import vdn_fp8._lib as L
+    M, pad = 3, 64
+    rng = np.random.default_rng(K)
+    hb = np.full((M, 2 * K + pad), 0x7FC0, np.uint16)
+    hb[:, :2 * K] = _randn_bits(rng, M, 2 * K, 2.0)
+    h = from_bits(hb, device)
+    y = torch.full((M, K + pad), 0x55, dtype=torch.uint8, device=device)
+    s = torch.empty(M, dtype=torch.float32, device=device)
+    L.check(L.load().vdn_fp8_swiglu_quantize_rows(h.data_ptr(), M, K, 2 * K + pad, y.data_ptr(), K + pad, s.data_ptr(),
+                                                  torch.cuda.current_stream().cuda_stream), "swiglu")
+    ya, sa = vdn_fp8.swiglu_quantize(h[:, :2 * K])
+    torch.cuda.synchronize()
+    assert torch.equal(y[:, :K], ya.view(torch.uint8)) and torch.equal(s, sa.reshape(-1))
+    assert bool((y[:, K:] == 0x55).all()), "wrote past K"
+    wy, ws = O.swiglu_quantize_rows(np.ascontiguousarray(hb[:, :2 * K]))
+    np.testing.assert_allclose(s.cpu().numpy(), ws, rtol=1e-6, atol=0)
+    assert np.mean(codes(ya) != wy) < 1e-3
+
+
 def test_quantize_rows_large_output(device):
     """An output beyond the last-level cache (>= 256 MiB of codes: the non-temporal store
     path) is bit-identical to quantizing the same rows in small batches (the cached store

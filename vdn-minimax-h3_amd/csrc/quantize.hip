@@ -946,7 +946,11 @@ __global__ __launch_bounds__(norm_row_waves(CPL, AFFINE) * kLanes) void k_norm_q
 
 // Wide rows (K > 8192 in the H3 FFN: 14336): WPR waves share a row, each holding
 // every WPR-th 1 KiB slice of it, so the binary32 activations fit in registers at
-// a useful occupancy; the row maximum is combined through LDS.
+// a useful occupancy; the row maximum is combined through LDS. Bound by HBM. With the
+// loads under per-chunk guards a wave had one or two chunks in flight and 86 VGPRs; all of
+// them first, unguarded, leave 69 at seven chunks per lane (seven workgroups per CU), so
+// that 1299 rows of H3's 14336 are one round: 29.3 -> 26.7 us; 13107 rows, at the rate of a
+// bare stream either way, 0.17 ms as before.
 template <int CPL, int WPR, bool NT>
 __global__ __launch_bounds__(kWavesPerBlock * kLanes) void k_swiglu_quant_split(
     const uint16_t* __restrict__ h, int64_t M, int64_t K, int64_t ldh,
@@ -959,19 +963,27 @@ __global__ __launch_bounds__(kWavesPerBlock * kLanes) void k_swiglu_quant_split(
     const int64_t row = (int64_t)blockIdx.x * (kWavesPerBlock / WPR) + wave / WPR;
     const bool valid = row < M;                      // no early return: the barrier below
     const int nch = (int)(K >> 3);
-    const int64_t r0 = valid ? row : 0;
-    const uint4* ar = reinterpret_cast<const uint4*>(h + r0 * ldh);
-    const uint4* gr = reinterpret_cast<const uint4*>(h + r0 * ldh + K);
+    // Every load first (chunks past K, and rows past M, outside the descriptors: zeros, no
+    // branch): the raw chunks take the registers that the activations then take over.
+    const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(h + (valid ? row : 0) * ldh), 0, valid ? (int)(K * 2) : 0, 0x00020000);
+    const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(h + (valid ? row : 0) * ldh + K), 0, valid ? (int)(K * 2) : 0, 0x00020000);
+    uint4 av[CPL], gv[CPL];
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+        const uint32_t off = (uint32_t)(part * kLanes + lane + kLanes * WPR * c) * 16;
+        av[c] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ar, off, 0, kBufferLoadOnce));
+        gv[c] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(gr, off, 0, kBufferLoadOnce));
+    }
+    __builtin_amdgcn_sched_barrier(0);
 
     float act[CPL][8];
     float amax = 0.0f;
     bool nan_seen = false;
 #pragma unroll
     for (int c = 0; c < CPL; ++c) {
-        const int idx = part * kLanes + lane + kLanes * WPR * c;
-        uint4 a = make_uint4(0u, 0u, 0u, 0u), g = a;
-        if (valid && idx < nch) { a = load_once(ar + idx); g = load_once(gr + idx); }
-        const uint32_t aw[4] = {a.x, a.y, a.z, a.w}, gw[4] = {g.x, g.y, g.z, g.w};
+        const uint32_t aw[4] = {av[c].x, av[c].y, av[c].z, av[c].w}, gw[4] = {gv[c].x, gv[c].y, gv[c].z, gv[c].w};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             act[c][2 * j] = swiglu(bf16_lo(aw[j]), bf16_lo(gw[j]));
@@ -1130,6 +1142,7 @@ extern "C" int vdn_fp8_swiglu_quantize_rows(const void* h, int64_t M, int64_t K,
         else hipLaunchKernelGGL((k_swiglu_quant_split<n, 4, false>), g1, block, 0, stream, hp, M, K, ldh, yp, ldy, scale);
         if (cpl <= 4) { VDN_SPLIT(4) }
         else if (cpl <= 6) { VDN_SPLIT(6) }
+        else if (nch <= 7 * 4 * kLanes) { VDN_SPLIT(7) }   // H3's 14336
         else { VDN_SPLIT(8) }
 #undef VDN_SPLIT
         return check_launch("swiglu_quantize_rows");
