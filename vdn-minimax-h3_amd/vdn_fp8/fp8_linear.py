@@ -50,7 +50,11 @@ def _stream(t):
 
 def ctypes_stream(device):
     """torch's current HIP stream on `device`, as the raw handle the C ABI takes."""
-    return torch.cuda.current_stream(device).cuda_stream
+    # (the handle alone: 0.1 us, where a Stream object to read it from takes 2.1 us)
+    index = device.index
+    if index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def _ptr(t):
@@ -67,6 +71,7 @@ def _aligned16(t):
 # reference's Triton kernels load any float type and compute in binary32 (fp8_linear.py:72);
 # float64 is refused here (its rows would be rounded to binary32 first).
 _DTYPES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16, torch.float32: _lib.DTYPE_F32}
+_FLOATS = tuple(_DTYPES)
 
 
 def _rows(x, dtypes=(torch.bfloat16,)):
@@ -130,7 +135,7 @@ def quantize_rows(x):
 
     Codes and scales are bit-identical to `quantize_rows_reference` (the reference's
     eager spelling, fp8_linear.py:132-135). Replaces fp8_linear.py:110-117."""
-    x = _rows(x, tuple(_DTYPES))
+    x = _rows(x, _FLOATS)
     M, K = x.shape
     y = torch.empty_like(x, dtype=FP8_DTYPE)
     scale = torch.empty(M, 1, device=x.device, dtype=torch.float32)
@@ -150,7 +155,7 @@ def swiglu_quantize(h):
     quantized row by row as in `quantize_rows`; returns e4m3 [M, K] and scales [M, 1].
     h may also be float16 or float32 (computed in binary32, as the reference's kernel
     loads it). Replaces fp8_linear.py:120-129."""
-    h = _rows(h, tuple(_DTYPES))
+    h = _rows(h, _FLOATS)
     M, K2 = h.shape
     if K2 % 2:
         raise ValueError(f"swiglu_quantize needs an even width, got {K2}")
@@ -374,20 +379,26 @@ class Fp8Linear(nn.Module):
             raise ValueError(f"the fused epilogues write bfloat16 (out_dtype={out_dtype})")
         if not x_fp8.is_cuda or x_fp8.dtype != FP8_DTYPE or x_fp8.dim() != 2:
             raise ValueError("x_fp8 must be a float8_e4m3fn [M, K] tensor on the GPU")
+        # (each read of a module's buffer goes through nn.Module.__getattr__: once per call)
+        weight, weight_scale, bias = self.weight_fp8, self.weight_scale, self.bias
         M, K = x_fp8.shape
-        N = self.weight_fp8.shape[0]
-        if K != self.weight_fp8.shape[1]:
-            raise ValueError(f"x has K={K}, the weight has K={self.weight_fp8.shape[1]}")
+        N, weight_k = weight.shape
+        if K != weight_k:
+            raise ValueError(f"x has K={K}, the weight has K={weight_k}")
         if x_scale.numel() != M or x_scale.dtype != torch.float32:
             raise ValueError("x_scale must be the fp32 [M, 1] rowwise scale (per-tensor scales are "
                              "the sm100 branch, not built for gfx950)")
         dev = x_fp8.device
-        if x_scale.device != dev or self.weight_fp8.device != dev:
+        if x_scale.device != dev or weight.device != dev:
             raise ValueError(f"x_fp8 ({dev}), x_scale ({x_scale.device}) and the fp8 weight "
-                             f"({self.weight_fp8.device}) must be on one device")
-        if x_fp8.stride(1) != 1:
+                             f"({weight.device}) must be on one device")
+        ldx, unit = x_fp8.stride()
+        if unit != 1:
             x_fp8 = x_fp8.contiguous()
-        x_fp8 = _aligned16(x_fp8)
+            ldx = x_fp8.stride(0)
+        aligned = _aligned16(x_fp8)
+        if aligned is not x_fp8:
+            x_fp8, ldx = aligned, aligned.stride(0)
         x_scale = _aligned16(x_scale.contiguous())
         lib = _lib.load()
         ws_bytes = gemm_workspace_bytes(M, N, K, dev)
@@ -398,13 +409,12 @@ class Fp8Linear(nn.Module):
             # GEMM's epilogue ([1111, 4100, 4112] float16: two passes over the output and
             # their launches less). Any other bias (one whose type promotes, that takes a
             # gradient, or that is no plain Parameter) is added as the reference's own op.
-            bias = self.bias
             fused = (type(bias) is nn.Parameter and bias.dtype == out_dtype and bias.shape == (N,)
                      and bias.device == dev and not (torch.is_grad_enabled() and bias.requires_grad))
             b = _aligned16(bias.detach().contiguous()) if fused else None
             out = torch.empty(M, N, device=dev, dtype=out_dtype)
-            _lib.check(lib.vdn_fp8_gemm_typed(_ptr(x_fp8), _ptr(x_scale), _ptr(self.weight_fp8),
-                                              _ptr(self.weight_scale), M, N, K, x_fp8.stride(0), K,
+            _lib.check(lib.vdn_fp8_gemm_typed(_ptr(x_fp8), _ptr(x_scale), _ptr(weight),
+                                              _ptr(weight_scale), M, N, K, ldx, K,
                                               _ptr(b), _DTYPES[out_dtype], _ptr(out), N, _ptr(ws), ws_bytes,
                                               _stream(x_fp8)),
                        "fp8 gemm")
@@ -413,7 +423,6 @@ class Fp8Linear(nn.Module):
         epi = _EPILOGUES.get(epilogue)
         if epi is None:
             raise ValueError(f"unknown epilogue {epilogue!r}")
-        bias = self.bias
         late_bias = None
         if bias is not None:
             if bias.numel() != N:
@@ -450,8 +459,8 @@ class Fp8Linear(nn.Module):
                 ldres = res.stride(0)
         elif gate is not None or residual is not None or gate_index is not None:
             raise ValueError('gate / gate_index / residual need epilogue="gate"')
-        _lib.check(lib.vdn_fp8_gemm_ws(_ptr(x_fp8), _ptr(x_scale), _ptr(self.weight_fp8),
-                                       _ptr(self.weight_scale), M, N, K, x_fp8.stride(0), K,
+        _lib.check(lib.vdn_fp8_gemm_ws(_ptr(x_fp8), _ptr(x_scale), _ptr(weight),
+                                       _ptr(weight_scale), M, N, K, ldx, K,
                                        _ptr(bias), epi, _ptr(g), _ptr(gi), grows, ldgate, _ptr(res), ldres,
                                        _ptr(out), N, _ptr(ws), ws_bytes, _stream(x_fp8)),
                    "fp8 gemm")
@@ -459,11 +468,12 @@ class Fp8Linear(nn.Module):
 
     def forward(self, x, **epilogue):
         shape = x.shape
-        rows = x.reshape(-1, shape[-1])
+        flat = x.dim() == 2   # already rows
+        rows = x if flat else x.reshape(-1, shape[-1])
         if "residual" in epilogue and epilogue["residual"] is not None:
             epilogue["residual"] = epilogue["residual"].reshape(rows.shape[0], -1)
         out = self.forward_quantized(*quantize_activation(rows), out_dtype=rows.dtype, **epilogue)
-        return out.reshape(*shape[:-1], -1)
+        return out if flat and shape[0] else out.reshape(*shape[:-1], -1)
 
 
 def _blocks_to_skip(model, skip_end_blocks):
