@@ -84,3 +84,27 @@ def test_typed_output_is_the_cast_and_the_add(device, dtype, M, N, K):
     assert f.forward_quantized(xq, xs, out_dtype=dtype).requires_grad
     f.bias = torch.nn.Parameter(f.bias.detach().double(), requires_grad=False)
     assert f.forward_quantized(xq, xs, out_dtype=dtype).dtype == torch.float64
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("M,N,K", [(1, 132, 1040), (65, 1028, 1136), (0, 64, 2064), (333, 260, 4112), (300, 512, 8208)])
+def test_forward_on_whole_lines(device, M, N, K, dtype):
+    """`Fp8Linear.forward` spaces the codes of such widths by whole 128-byte lines: the output is
+    bit for bit that of contiguous codes, also where every byte past a row's K is a NaN code."""
+    g = torch.Generator(device=device).manual_seed(K + M)
+    lin = torch.nn.Linear(K, N, dtype=dtype, device=device)
+    f = vdn_fp8.Fp8Linear(lin)
+    x = torch.randn(2, M, K, device=device, generator=g).to(dtype)   # (three dimensions: also without rows)
+    with torch.no_grad():
+        if M == 0:
+            with pytest.raises(RuntimeError):
+                f(x[0])          # as torch's reshape to (0, -1) refuses it
+            return
+        q, s = vdn_fp8.quantize_activation(x.reshape(-1, K))
+        want = f.forward_quantized(q, s, out_dtype=dtype)
+        padded = torch.full((2 * M, -(-K // 128) * 128), 0x7F, device=device, dtype=torch.uint8)
+        padded[:, :K] = q.view(torch.uint8)
+        got = f.forward_quantized(padded.view(torch.float8_e4m3fn)[:, :K], s, out_dtype=dtype)
+        bits = torch.int32 if dtype == torch.float32 else torch.int16
+        assert torch.equal(got.view(bits), want.view(bits))
+        assert torch.equal(f(x).reshape(-1, N).view(bits), want.view(bits))
