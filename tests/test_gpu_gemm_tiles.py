@@ -46,7 +46,8 @@ def _pad(t, *shape):
     (2317, 5376, 256, "gelu"),        # 224-row tiles of the persistent kernel
     (2317, 5376, 512, "rows"),
     (1928, 4096, 512, "bias"),        # 128 tiles as halves
-    (4000, 4168, 2048, "rows"),       # one round and a last one in quarters, columns past N
+    (4000, 4168, 2048, "rows"),       # one round and a last one in eighths, columns past N
+    (4000, 4704, 2048, "rows"),       # one round and a last one in quarters
 ])
 def test_tile_shapes_give_the_same_bits(device, M, N, K, epi):
     print(f"gemm tiles [{M}, {N}, {K}] {epi}", flush=True)

@@ -898,6 +898,11 @@ GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int cus, bool split_ok, bool
                 }
                 if (2 * R <= cus) take(base + part_us(tile_of(8, 4), 2.0 * (double)R) + 1.0, {true, 8, (int)(T - R), 0, 0, 8, 4});
                 if (4 * R <= cus) take(base + part_us(tile_of(4, 4), 4.0 * (double)R) + 1.0, {true, 8, (int)(T - R), 0, 0, 4, 4});
+                // (a last round of so few tiles is bound by one part's chain of K blocks, and this part's
+                // block is the shortest: [4680, 13824, 5120], two tiles left of 1026, 244.6 us as
+                // quarters, 238.8 as eighths. Longer rows split along K.)
+                if (8 * R <= cus && K < kSplitMinK)
+                    take(base + part_us(tile_of(4, 2), 8.0 * (double)R) + 1.0, {true, 8, (int)(T - R), 0, 0, 4, 2});
             }
             take(base + round_us((double)R / cus) + (full ? 0.0 : 5.0), whole);
         }
