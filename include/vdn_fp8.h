@@ -37,7 +37,7 @@
 extern "C" {
 #endif
 
-#define VDN_FP8_ABI_VERSION 5
+#define VDN_FP8_ABI_VERSION 6
 
 /* status codes */
 #define VDN_FP8_OK 0
@@ -220,6 +220,22 @@ int vdn_fp8_gemm(const void *xq, const float *x_scale, const void *wq, const flo
  *           src/models/ops/fp8_linear.py:272); the query for the next call.
  */
 int vdn_fp8_gemm_workspace_size(int64_t M, int64_t N, int64_t K, int64_t *bytes);
+
+/*
+ * Which kernels an [M, N, K] GEMM runs, for tests and tuning (host only; no GPU needed
+ * when cus > 0). rows16: a bf16 output whose rows, with the gate's and the residual's,
+ * take 16-byte accesses; split_ok: a workspace is given; cus: compute units, 0 = the
+ * current device's. plan[0..5]:
+ *   [0] rows of the persistent kernel's tiles (256 or 224; 256 channels each), 0: not used
+ *   [1] tiles it runs whole
+ *   [2] K slices of each 256 x 256 tile past those, [3] their number in all (0: no split)
+ *   [4] channels and [5] tokens of the small tiles that do the rest, or with plan[0] = 0
+ *       all of it (0: none)
+ * us, if not NULL, receives the estimate in microseconds by which it was chosen.
+ * Replaces: nothing in the reference (cuBLASLt's heuristics are not visible there).
+ */
+int vdn_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, int rows16, int split_ok, int cus,
+                      int32_t *plan, double *us);
 
 /*
  * vdn_fp8_gemm with a caller-provided split-K workspace (device memory, 16-byte

@@ -60,3 +60,14 @@ def same_codes(got, want):
     want = np.asarray(want, np.uint8)
     nan = lambda c: (c & 0x7F) == 0x7F
     return (got == want) | (nan(got) & nan(want))
+
+
+def gemm_plan(M, N, K, rows16=True, split=False, cus=256):
+    """vdn_fp8_gemm_plan: (tile rows, whole tiles, K slices per tile, split units, part
+    channels, part tokens) on a part of `cus` compute units (0: the current device)."""
+    import ctypes
+
+    import vdn_fp8._lib as L
+    plan = (ctypes.c_int32 * 6)()
+    L.check(L.load().vdn_fp8_gemm_plan(M, N, K, int(rows16), int(split), cus, plan, None), "gemm_plan")
+    return tuple(plan)

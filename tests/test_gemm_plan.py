@@ -1,0 +1,54 @@
+"""The GEMM's plan (vdn_fp8_gemm_plan; no GPU needed): which kernels run a shape."""
+import ctypes
+import random
+
+import pytest
+
+from conftest import gemm_plan
+
+CUS = 256
+
+
+def _shapes(n, seed):
+    rng = random.Random(seed)
+    lg = lambda a, b: int(a * (b / a) ** rng.random())
+    return [(lg(1, 40000), max(4, lg(4, 40000) // 4 * 4), max(16, lg(16, 40000) // rng.choice([16, 256]) * 16))
+            for _ in range(n)] + [(lg(1, 40000), lg(64, 10000) * 4, 256 * lg(1, 128)) for _ in range(n)]
+
+
+@pytest.mark.parametrize("rows16,split", [(True, True), (True, False), (False, True), (False, False)])
+def test_a_plan_covers_every_tile(rows16, split):
+    """Whole tiles, split tiles and parts add up to the output, within what each kernel takes."""
+    for M, N, K in _shapes(400, 1):
+        rows, whole, slices, units, a, b = gemm_plan(M, N, K, rows16, split)
+        case = (M, N, K, rows16, split, rows, whole, slices, units, a, b)
+        if rows == 0:
+            assert whole == units == 0 and a and b, case
+            continue
+        assert K % 256 == 0 and rows in ((224, 256) if rows16 else (256,)), case
+        tiles = -(-M // rows) * -(-N // 256)
+        if units:
+            assert split and K >= 8192 and not a and slices >= 2 and K // 256 >= slices, case
+            assert whole + units // slices == tiles and units % slices == 0 and units <= CUS, case
+        elif a:
+            parts = (tiles - whole) * (256 // a) * (256 // b)
+            assert rows == 256 and a in (128, 256) and b in (64, 128) and 0 < parts <= CUS, case
+        else:
+            assert whole == tiles, case
+
+
+def test_large_shapes_run_whole_tiles():
+    assert gemm_plan(32760, 15360, 5120)[:2] == (256, 7680)
+    assert gemm_plan(32760, 15360, 5120, rows16=False)[:2] == (256, 7680)
+
+
+def test_query_refusals():
+    import vdn_fp8._lib as L
+    lib = L.load()
+    plan = (ctypes.c_int32 * 6)()
+    us = ctypes.c_double()
+    assert lib.vdn_fp8_gemm_plan(1, 4, 16, 1, 0, CUS, None, None) == L.EINVAL
+    assert lib.vdn_fp8_gemm_plan(0, 4, 16, 1, 0, CUS, plan, None) == L.EINVAL
+    assert lib.vdn_fp8_gemm_plan(1, 4, 16, 1, 0, -1, plan, None) == L.EINVAL
+    assert lib.vdn_fp8_gemm_plan(1 << 40, 1 << 20, 16, 1, 0, CUS, plan, None) == L.EINVAL
+    assert lib.vdn_fp8_gemm_plan(1, 4, 16, 1, 0, CUS, plan, ctypes.byref(us)) == L.OK and us.value > 0

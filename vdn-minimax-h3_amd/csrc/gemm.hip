@@ -860,7 +860,7 @@ struct GemmPlan {
 // [821, 5376, 5120], 84 tiles of 256 x 256 on 256 CUs: 47 us there, 27.3 us as 196 tiles of
 // 128 x 192; [300, 5376, 5120] 31 -> 17.6 us; [1299, 28672, 5376] 180 -> 172 us with 224-row
 // tiles (the same 672 tiles, an eighth less of each); [4680, 13824, 5120] 260 -> 246 us.
-GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int cus, bool split_ok, bool rows224_ok)
+GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int cus, bool split_ok, bool rows224_ok, double* est = nullptr)
 {
     const double nk = (double)((K + mainloop::BK - 1) / mainloop::BK);
     int count = 0;
@@ -891,10 +891,14 @@ GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int cus, bool split_ok, bool
             if (xb == 8) {
                 const int64_t S = 2 * R <= cus ? std::min<int64_t>(cus / R, (int64_t)nk / kSplitMinBlocks) : 0;
                 if (split_ok && K >= kSplitMinK && S >= 2) {
+                    const double split_us = base + nk / (double)S * 1.2 + 15.0 + 0.05 * (double)(R * S);
                     const GemmPlan split{true, 8, (int)(T - R), (int)S, (int)(R * S), 0, 0};
                     // (at most 16 tiles over such rows: callers hold workspaces for them)
-                    if (T <= 16) return split;
-                    take(base + nk / (double)S * 1.2 + 15.0 + 0.05 * (double)(R * S), split);
+                    if (T <= 16) {
+                        if (est) *est = split_us;
+                        return split;
+                    }
+                    take(split_us, split);
                 }
                 if (2 * R <= cus) take(base + part_us(tile_of(8, 4), 2.0 * (double)R) + 1.0, {true, 8, (int)(T - R), 0, 0, 8, 4});
                 if (4 * R <= cus) take(base + part_us(tile_of(4, 4), 4.0 * (double)R) + 1.0, {true, 8, (int)(T - R), 0, 0, 4, 4});
@@ -914,6 +918,7 @@ GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int cus, bool split_ok, bool
         us += units % cus ? part_us(t, (double)(units % cus)) : 5.0;
         take(K >= kSplitMinK ? 1.1 * us : us, {false, 0, 0, 0, 0, t.a, t.b});
     }
+    if (est) *est = best_us;
     return best;
 }
 
@@ -1062,6 +1067,20 @@ extern "C" int vdn_fp8_gemm_workspace_size(int64_t M, int64_t N, int64_t K, int6
 {
     if (!bytes) return set_error(VDN_FP8_EINVAL, "gemm_workspace_size: null pointer");
     return gemm_workspace_bytes(M, N, K, bytes);
+}
+
+extern "C" int vdn_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, int rows16, int split_ok, int cus, int32_t* plan, double* us)
+{
+    if (!plan) return set_error(VDN_FP8_EINVAL, "gemm_plan: null pointer");
+    if (M <= 0 || N <= 0 || K <= 0 || cus < 0) return set_error(VDN_FP8_EINVAL, "gemm_plan: sizes must be positive");
+    if (((M + BM - 1) / BM) * ((N + BN - 1) / BN) > (int64_t)INT32_MAX / 16)
+        return set_error(VDN_FP8_EINVAL, "gemm_plan: problem too large");
+    if (cus == 0 && (cus = device_cus()) <= 0)
+        return set_error(VDN_FP8_ELAUNCH, "gemm_plan: cannot query the device's compute units");
+    const GemmPlan p = plan_gemm(M, N, K, cus, split_ok != 0, rows16 != 0, us);
+    const int32_t v[6] = {p.main ? 32 * p.xb : 0, p.main ? p.t_main : 0, p.units ? p.splits : 0, p.units, 32 * p.a, 32 * p.b};
+    for (int i = 0; i < 6; ++i) plan[i] = v[i];
+    return VDN_FP8_OK;
 }
 
 extern "C" int vdn_fp8_gemm_ws(const void* xq, const float* x_scale, const void* wq, const float* w_scale, int64_t M,

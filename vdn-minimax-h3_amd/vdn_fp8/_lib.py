@@ -12,7 +12,7 @@ import os
 
 from .build import CSRC, INCLUDE, LIB_PATH, compiler_id, source_manifest
 
-ABI_VERSION = 5
+ABI_VERSION = 6
 
 OK, EINVAL, ELAUNCH = 0, 1, 2
 EPI_NONE, EPI_GELU_TANH, EPI_GATE, EPI_F32 = 0, 1, 2, 3
@@ -36,6 +36,7 @@ EXPORTS = (
     ("vdn_fp8_gemm", _I32, [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _I32, _P, _P, _I64, _I64,
                             _P, _I64, _P, _I64, _P]),
     ("vdn_fp8_gemm_workspace_size", _I32, [_I64, _I64, _I64, _P]),
+    ("vdn_fp8_gemm_plan", _I32, [_I64, _I64, _I64, _I32, _I32, _I32, _P, _P]),
     ("vdn_fp8_gemm_ws", _I32, [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _I32, _P, _P, _I64, _I64,
                                _P, _I64, _P, _I64, _P, _I64, _P]),
     ("vdn_fp8_gemm_typed", _I32, [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _I32, _P, _I64, _P, _I64, _P]),
