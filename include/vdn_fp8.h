@@ -224,7 +224,8 @@ int vdn_fp8_gemm_workspace_size(int64_t M, int64_t N, int64_t K, int64_t *bytes)
 /*
  * Which kernels an [M, N, K] GEMM runs, for tests and tuning (host only; no GPU needed
  * when cus > 0). rows16: a bf16 output whose rows, with the gate's and the residual's,
- * take 16-byte accesses; split_ok: a workspace is given; cus: compute units, 0 = the
+ * take 16-byte accesses; workspace: one of at
+ * least the size query's answer is given; cus: compute units, 0 = the
  * current device's. plan[0..5]:
  *   [0] rows of the persistent kernel's tiles (256 or 224; 256 channels each), 0: not used
  *   [1] tiles it runs whole
@@ -234,7 +235,7 @@ int vdn_fp8_gemm_workspace_size(int64_t M, int64_t N, int64_t K, int64_t *bytes)
  * us, if not NULL, receives the estimate in microseconds by which it was chosen.
  * Replaces: nothing in the reference (cuBLASLt's heuristics are not visible there).
  */
-int vdn_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, int rows16, int split_ok, int cus,
+int vdn_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, int rows16, int workspace, int cus,
                       int32_t *plan, double *us);
 
 /*

@@ -37,6 +37,18 @@ def test_a_plan_covers_every_tile(rows16, split):
             assert whole == tiles, case
 
 
+def test_the_size_query_answers_for_every_epilogue():
+    """The workspace is sized by M, N and K alone; a call whose rows take the general epilogue
+    (binary16 or binary32 output, rows that are not 16-byte) needs no more than that."""
+    shapes = [(M, N, K) for M in range(1, 5000, 37) for N in (512, 4100, 5376, 15360, 28672) for K in (8192, 14336)]
+    apart = 0
+    for M, N, K in shapes + [(2817, 28672, 8192), (2912, 28672, 8192), (3329, 28672, 8192)]:
+        answer, need = gemm_plan(M, N, K, True, True)[3], gemm_plan(M, N, K, False, True)[3]
+        assert need <= answer, (M, N, K, need, answer)
+        apart += gemm_plan(M, N, K, True, True) != gemm_plan(M, N, K, False, True)
+    assert apart
+
+
 def test_large_shapes_run_whole_tiles():
     assert gemm_plan(32760, 15360, 5120)[:2] == (256, 7680)
     assert gemm_plan(32760, 15360, 5120, rows16=False)[:2] == (256, 7680)

@@ -75,3 +75,28 @@ def test_tile_shapes_give_the_same_bits(device, M, N, K, epi):
     torch.cuda.synchronize()
     bits = torch.int32 if epi == "f32" else torch.int16
     assert torch.equal(got.view(bits), want.contiguous().view(bits))
+
+
+@pytest.mark.parametrize("M,N,K,out", [(2817, 28672, 8192, "f16"), (3329, 28676, 8192, "bf16")])
+def test_the_answered_workspace_is_enough(device, M, N, K, out):
+    """A workspace of the queried size (at least 16 bytes, so that a pointer is given) serves rows
+    that take the general epilogue too, where the query assumes 16-byte rows."""
+    print(f"gemm workspace [{M}, {N}, {K}] {out}", flush=True)
+    g = torch.Generator(device=device).manual_seed(M)
+    code = lambda *s: torch.randint(0, 120, s, device=device, generator=g, dtype=torch.uint8).view(torch.float8_e4m3fn)
+    xq, wq = code(M, K), code(N, K)
+    sx, sw = (1e-4 * torch.rand(n, device=device, generator=g) for n in (M, N))
+    ws = torch.empty(max(16, vdn_fp8.fp8_linear.gemm_workspace_bytes(M, N, K, device)), device=device, dtype=torch.uint8)
+    st = torch.cuda.current_stream().cuda_stream
+    lib, outs = L.load(), []
+    for w, size in ((ws.data_ptr(), ws.numel()), (None, 0)):
+        o = torch.empty(M, N, device=device, dtype=torch.float16 if out == "f16" else torch.bfloat16)
+        a = (xq.data_ptr(), sx.data_ptr(), wq.data_ptr(), sw.data_ptr(), M, N, K, K, K)
+        if out == "f16":
+            L.check(lib.vdn_fp8_gemm_typed(*a, None, L.DTYPE_F16, o.data_ptr(), N, w, size, st), "gemm")
+        else:
+            L.check(lib.vdn_fp8_gemm_ws(*a, None, L.EPI_NONE, None, None, 0, 0, None, 0, o.data_ptr(), N, w, size, st), "gemm")
+        outs.append(o)
+    torch.cuda.synchronize()
+    if ws.numel() == 16:
+        assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))   # no split either way

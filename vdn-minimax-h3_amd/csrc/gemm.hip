@@ -922,6 +922,16 @@ GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int cus, bool split_ok, bool
     return best;
 }
 
+// The plan of a call. The workspace's size is asked for by M, N and K alone, as for 16-byte rows, so
+// other rows split only where that answer holds the partial sums: a workspace of the answered
+// size is never too small. ([2900, 28672, 8192]: 224-row tiles and no workspace for 16-byte rows,
+// where other rows alone would be estimated fastest as 256 slices, 64 MiB.)
+GemmPlan plan_call(int64_t M, int64_t N, int64_t K, int cus, bool workspace, bool rows16, double* est = nullptr)
+{
+    const bool split_ok = workspace && K >= kSplitMinK && (rows16 || plan_gemm(M, N, K, cus, true, true).units);
+    return plan_gemm(M, N, K, cus, split_ok, rows16, est);
+}
+
 }  // namespace
 
 int launch_gated_residual(const uint16_t* residual, int64_t ldr, const uint16_t* gate, int64_t ldgate,
@@ -937,7 +947,7 @@ int gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t* bytes)
     if (cus <= 0) return set_error(VDN_FP8_ELAUNCH, "gemm: cannot query the device's compute units");
     const int64_t T = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     if (T > (int64_t)INT32_MAX / 16) return VDN_FP8_OK;
-    *bytes = (int64_t)plan_gemm(M, N, K, cus, true, true).units * kUnitFloats * (int64_t)sizeof(float);
+    *bytes = (int64_t)plan_call(M, N, K, cus, true, true).units * kUnitFloats * (int64_t)sizeof(float);
     return VDN_FP8_OK;
 }
 
@@ -991,7 +1001,7 @@ int gemm_launch(const void* xq, const float* x_scale, const void* wq, const floa
                         (!residual || (aligned(residual, 16) && ldres % 8 == 0));
     const bool rows31 = rows16 && (!residual || (int64_t)BM * ldres * 2 <= kMax) && gate_rows * ldgate * 2 <= kMax;
     const bool fast = out16 && epilogue != VDN_FP8_EPI_F32 && (!gated || gate_broadcast || rows31);
-    const GemmPlan plan = plan_gemm(M, N, K, cus, ws != nullptr, fast);
+    const GemmPlan plan = plan_call(M, N, K, cus, ws != nullptr, fast);
     GemmArgs p{(const uint8_t*)xq, x_scale, (const uint8_t*)wq, w_scale, M, N, K, ldx, ldw,
                (const uint16_t*)bias, (const uint16_t*)gate, gate_index, gate_rows, ldgate,
                (const uint16_t*)residual, ldres, (uint16_t*)out, ldo,
@@ -1069,7 +1079,8 @@ extern "C" int vdn_fp8_gemm_workspace_size(int64_t M, int64_t N, int64_t K, int6
     return gemm_workspace_bytes(M, N, K, bytes);
 }
 
-extern "C" int vdn_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, int rows16, int split_ok, int cus, int32_t* plan, double* us)
+extern "C" int vdn_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, int rows16, int workspace, int cus, int32_t* plan,
+                                 double* us)
 {
     if (!plan) return set_error(VDN_FP8_EINVAL, "gemm_plan: null pointer");
     if (M <= 0 || N <= 0 || K <= 0 || cus < 0) return set_error(VDN_FP8_EINVAL, "gemm_plan: sizes must be positive");
@@ -1077,7 +1088,7 @@ extern "C" int vdn_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, int rows16, in
         return set_error(VDN_FP8_EINVAL, "gemm_plan: problem too large");
     if (cus == 0 && (cus = device_cus()) <= 0)
         return set_error(VDN_FP8_ELAUNCH, "gemm_plan: cannot query the device's compute units");
-    const GemmPlan p = plan_gemm(M, N, K, cus, split_ok != 0, rows16 != 0, us);
+    const GemmPlan p = plan_call(M, N, K, cus, workspace != 0, rows16 != 0, us);
     const int32_t v[6] = {p.main ? 32 * p.xb : 0, p.main ? p.t_main : 0, p.units ? p.splits : 0, p.units, 32 * p.a, 32 * p.b};
     for (int i = 0; i < 6; ++i) plan[i] = v[i];
     return VDN_FP8_OK;
