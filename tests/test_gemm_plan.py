@@ -54,6 +54,17 @@ def test_large_shapes_run_whole_tiles():
     assert gemm_plan(32760, 15360, 5120, rows16=False)[:2] == (256, 7680)
 
 
+@pytest.mark.parametrize("M,N,K,rows16,want", [
+    (2074, 10400, 256, True, (224, 410, 0, 0, 0, 0)),       # 19.5 us; 26.3 on the tile kernel's 256 x 128
+    (3891, 2704, 256, True, (224, 198, 0, 0, 0, 0)),        # 16.7 us; 19.7 as 128 x 192
+    (10329, 2232, 1024, False, (256, 256, 0, 0, 256, 128)), # 40.3 us; 44.7 as 256 x 128 throughout
+    (1304, 2272, 1024, True, (0, 0, 0, 0, 128, 96)),        # 9.9 us; 12.1 as 192 x 96
+])
+def test_short_rows_count_the_epilogue(M, N, K, rows16, want):
+    """At a K of a few blocks most of a round is its epilogue (times: one MI355X)."""
+    assert gemm_plan(M, N, K, rows16) == want
+
+
 def test_query_refusals():
     import vdn_fp8._lib as L
     lib = L.load()

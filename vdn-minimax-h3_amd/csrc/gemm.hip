@@ -847,19 +847,25 @@ struct GemmPlan {
     int xb, t_main, splits, units, a, b;
 };
 
-// The plan of a shape, by the estimated time of each way to run it. Per 128-byte K block,
-// in us on one MI355X (fits of measured times over M 64 .. 3120 and the layers' widths,
-// within 15%; the choice among them cost 3% on average against the best of each):
+// The plan of a shape, by the estimated time of each way to run it, from rates measured on one
+// MI355X, in us. Per 128-byte K block:
 //   persistent kernel: a round of 256-row tiles 1.0 on a few compute units, 1.43 on all of
 //     them (the part's power), of 224-row tiles 0.98 to 1.33;
 //   tile kernel: kTiles' `alone`, or what the copies of all its tiles take at 16 TB/s out of
 //     the L2s if that is longer; `busy` for a whole round of many; the weight's bytes at
 //     4.9 TB/s bound the shortest calls;
-//   a split: its slices' blocks at 1.2, and 15 us + 0.05 per slice for the partial sums and
+//   a split: its slices' blocks at 1.2, and 22 us + 0.05 per slice for the partial sums and
 //     their reduction.
+// And per round the epilogue with its stores, which at a K of a few blocks is most of the time:
+// 5.8 to 7.9 for 256-row tiles, 0.155 to 0.26 per 32 x 32 outputs of a tile of the tile kernel.
+// Without that term shapes of K <= 1024 went to the tile kernel where the persistent one is
+// faster: [2074, 10400, 256] 26.3 against 19.5 us, [1304, 2272, 1024] 12.1 against 9.9.
+// Over 2143 drawn shapes (M 1 .. 16384, N 64 .. 30000, K 128 .. 16384, every epilogue, each way
+// timed) the choice costs 1.5% on average against the best way, 9% at the 95th percentile;
+// half of the estimates are within 9% of the time, nine tenths between 0.75 and 1.24 of it.
 // [821, 5376, 5120], 84 tiles of 256 x 256 on 256 CUs: 47 us there, 27.3 us as 196 tiles of
-// 128 x 192; [300, 5376, 5120] 31 -> 17.6 us; [1299, 28672, 5376] 180 -> 172 us with 224-row
-// tiles (the same 672 tiles, an eighth less of each); [4680, 13824, 5120] 260 -> 246 us.
+// 192 channels x 128 tokens; [300, 5376, 5120] 31 -> 17.6 us; [1299, 28672, 5376] 180 -> 172 us
+// with 224-row tiles (the same 672 tiles, an eighth less of each); [4680, 13824, 5120] 260 -> 246.
 GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int cus, bool split_ok, bool rows224_ok, double* est = nullptr)
 {
     const double nk = (double)((K + mainloop::BK - 1) / mainloop::BK);
@@ -868,7 +874,8 @@ GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int cus, bool split_ok, bool
     const double floor_us = (double)N * (double)K / 4.9e6 + 3.0;
     auto part_us = [&](const GemmTile& t, double units) {   // at most one round of them
         const double copies = units * (t.a + t.b) * 4096e-6 / 16.0;
-        return std::max(nk * std::max(t.alone, copies) + 4.5, floor_us);
+        const double epilogue = (0.155 + 0.05 * std::min(1.0, units / cus)) * t.a * t.b;
+        return std::max(nk * std::max(t.alone, copies) + 3.2 + epilogue, floor_us);
     };
     auto tile_of = [&](int a, int b) {
         int i = 0;
@@ -884,14 +891,16 @@ GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int cus, bool split_ok, bool
         const int64_t tn = (N + BN - 1) / BN;
         for (int xb = 8; xb >= (rows224_ok ? 7 : 8); --xb) {
             const int64_t T = ((M + 32 * xb - 1) / (32 * xb)) * tn, full = T / cus, R = T % cus;
-            auto round_us = [&](double load) { return nk * (xb == 8 ? 1.0 + 0.43 * load : 0.98 + 0.35 * load); };
+            auto round_us = [&](double load) {
+                return nk * (xb == 8 ? 1.0 + 0.43 * load : 0.98 + 0.35 * load) + (xb == 8 ? 5.8 + 2.1 * load : 4.8 + 1.7 * load);
+            };
             const double base = (double)full * round_us(1.0) + (full ? 5.0 : 0.0);
             const GemmPlan whole{true, xb, (int)T, 0, 0, 0, 0};
             if (R == 0) { take(base, whole); continue; }
             if (xb == 8) {
                 const int64_t S = 2 * R <= cus ? std::min<int64_t>(cus / R, (int64_t)nk / kSplitMinBlocks) : 0;
                 if (split_ok && K >= kSplitMinK && S >= 2) {
-                    const double split_us = base + nk / (double)S * 1.2 + 15.0 + 0.05 * (double)(R * S);
+                    const double split_us = base + nk / (double)S * 1.2 + 21.9 + 0.05 * (double)(R * S);
                     const GemmPlan split{true, 8, (int)(T - R), (int)S, (int)(R * S), 0, 0};
                     // (at most 16 tiles over such rows: callers hold workspaces for them)
                     if (T <= 16) {
@@ -900,13 +909,13 @@ GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int cus, bool split_ok, bool
                     }
                     take(split_us, split);
                 }
-                if (2 * R <= cus) take(base + part_us(tile_of(8, 4), 2.0 * (double)R) + 1.0, {true, 8, (int)(T - R), 0, 0, 8, 4});
-                if (4 * R <= cus) take(base + part_us(tile_of(4, 4), 4.0 * (double)R) + 1.0, {true, 8, (int)(T - R), 0, 0, 4, 4});
+                if (2 * R <= cus) take(base + part_us(tile_of(8, 4), 2.0 * (double)R) + 0.4, {true, 8, (int)(T - R), 0, 0, 8, 4});
+                if (4 * R <= cus) take(base + part_us(tile_of(4, 4), 4.0 * (double)R) + 0.4, {true, 8, (int)(T - R), 0, 0, 4, 4});
                 // (a last round of so few tiles is bound by one part's chain of K blocks, and this part's
                 // block is the shortest: [4680, 13824, 5120], two tiles left of 1026, 244.6 us as
                 // quarters, 238.8 as eighths. Longer rows split along K.)
                 if (8 * R <= cus && K < kSplitMinK)
-                    take(base + part_us(tile_of(4, 2), 8.0 * (double)R) + 1.0, {true, 8, (int)(T - R), 0, 0, 4, 2});
+                    take(base + part_us(tile_of(4, 2), 8.0 * (double)R) + 0.4, {true, 8, (int)(T - R), 0, 0, 4, 2});
             }
             take(base + round_us((double)R / cus) + (full ? 0.0 : 5.0), whole);
         }
@@ -914,7 +923,7 @@ GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int cus, bool split_ok, bool
     for (int i = 0; i < count; ++i) {
         const GemmTile& t = tiles[i];
         const int64_t units = ((M + 32 * t.b - 1) / (32 * t.b)) * ((N + 32 * t.a - 1) / (32 * t.a));
-        double us = (double)(units / cus) * nk * t.busy;
+        double us = (double)(units / cus) * (nk * t.busy + 0.26 * t.a * t.b);
         us += units % cus ? part_us(t, (double)(units % cus)) : 5.0;
         take(K >= kSplitMinK ? 1.1 * us : us, {false, 0, 0, 0, 0, t.a, t.b});
     }
