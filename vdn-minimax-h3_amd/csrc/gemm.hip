@@ -854,7 +854,7 @@ struct GemmPlan {
 //   tile kernel: kTiles' `alone`, or what the copies of all its tiles take at 16 TB/s out of
 //     the L2s if that is longer; `busy` for a whole round of many; the weight's bytes at
 //     4.9 TB/s bound the shortest calls;
-//   a split: its slices' blocks at 1.2, and 22 us + 0.05 per slice for the partial sums and
+//   a split: its slices' blocks at 1.2, and 14 us + 0.07 per slice for the partial sums and
 //     their reduction.
 // And per round the epilogue with its stores, which at a K of a few blocks is most of the time:
 // 5.8 to 7.9 for 256-row tiles, 0.155 to 0.26 per 32 x 32 outputs of a tile of the tile kernel.
@@ -900,7 +900,7 @@ GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int cus, bool split_ok, bool
             if (xb == 8) {
                 const int64_t S = 2 * R <= cus ? std::min<int64_t>(cus / R, (int64_t)nk / kSplitMinBlocks) : 0;
                 if (split_ok && K >= kSplitMinK && S >= 2) {
-                    const double split_us = base + nk / (double)S * 1.2 + 21.9 + 0.05 * (double)(R * S);
+                    const double split_us = base + nk / (double)S * 1.2 + 14.0 + 0.07 * (double)(R * S);
                     const GemmPlan split{true, 8, (int)(T - R), (int)S, (int)(R * S), 0, 0};
                     // (at most 16 tiles over such rows: callers hold workspaces for them)
                     if (T <= 16) {
