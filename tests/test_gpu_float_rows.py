@@ -56,6 +56,20 @@ def test_float_rows_bit_exact(device, dtype, widths, weight):
         assert np.array_equal(s.cpu().numpy().reshape(-1).view(np.uint32), want_s.view(np.uint32))
 
 
+def test_more_rows_than_workgroups_in_a_launch(device):
+    """2^24 rows and more, which a launch of one 256-thread workgroup per row cannot hold."""
+    M, K = (1 << 24) + 5, 8
+    print(f"float rows [{M}, {K}]", flush=True)
+    x = torch.zeros(M, K, device=device, dtype=torch.float16)
+    rows = torch.tensor([0, 1, 255, 1 << 16, (1 << 24) - 1, 1 << 24, M - 1], device=device)
+    x[rows] = torch.randn(rows.numel(), K, device=device, generator=torch.Generator(device=device).manual_seed(3)).half()
+    q, s = vdn_fp8.quantize_rows(x)
+    want_q, want_s = O.quantize_rows_float(x[rows].cpu().numpy())
+    assert same_codes(codes(q[rows]), want_q).all()
+    assert np.array_equal(s[rows].cpu().numpy().reshape(-1).view(np.uint32), want_s.view(np.uint32))
+    assert int((s != s[2 ** 20 + 1]).sum()) == rows.numel() and int((q.view(torch.uint8).sum(1) != 0).sum()) == rows.numel()
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("M,N,K", [(1, 4, 16), (77, 260, 400), (700, 1032, 2048), (4096, 4096, 512), (520, 1028, 8192)])
 def test_typed_output_is_the_cast_and_the_add(device, dtype, M, N, K):

@@ -1320,14 +1320,15 @@ int check_typed_rows(const char* what, const void* x, int dtype, int64_t M, int6
 }
 
 // The float row quantizers by the row's 16-byte pieces: 256 per workgroup and step, up to 16
-// steps in registers, past that the two sweeps.
+// steps in registers, past that (and past the rows that fit one launch of a workgroup each)
+// the two sweeps.
 template <typename T, bool kWeight>
 int launch_rowquant_float(const char* what, const T* x, int64_t M, int64_t K, int64_t ldx, uint8_t* y, int64_t ldy,
                           float* scale, hipStream_t stream)
 {
     const dim3 block(kWavesPerBlock * kLanes);
     const int64_t per = (K / FloatRow<T>::kPer + kWavesPerBlock * kLanes - 1) / (kWavesPerBlock * kLanes);
-    if (per > 16 || M > 0x7fffffff) {
+    if (per > 16 || M >= 1 << 24) {   // (a launch takes fewer than 2^32 work-items: 2^24 workgroups)
         const dim3 grid((unsigned)((M + kWavesPerBlock - 1) / kWavesPerBlock));
         hipLaunchKernelGGL((k_rowquant_float_wide<T, kWeight>), grid, block, 0, stream, x, M, K, ldx, y, ldy, scale);
         return check_launch(what);
