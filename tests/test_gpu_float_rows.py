@@ -1,7 +1,7 @@
 """GPU: float16 / float32 rows through the one-read quantizers and the GEMM's typed output.
 
-The quantizer's row widths cover each register count's edges and the two-sweep kernel past
-them; besides ordinary values every row holds elements at, one ulp below and one above each
+The quantizer's row widths cover each register count's edges and the two-sweep kernel below
+and past them; besides ordinary values every row holds elements at, one ulp below and one above each
 e4m3 rounding boundary times the row's scale, where a quotient off by one ulp would change
 the code. The GEMM's float16 / float32 output with its bias must give the bits of the binary32
 product followed by torch's own cast and add."""
@@ -38,8 +38,8 @@ def _row(rng, K, dtype, amax):
 
 @pytest.mark.parametrize("weight", [False, True])
 @pytest.mark.parametrize("dtype,widths", [
-    (torch.float32, (8, 1016, 1024, 1032, 4096, 5120, 8192, 12296, 16384, 16392)),
-    (torch.float16, (8, 2040, 2048, 2056, 8192, 13824, 24576, 32768, 32776))])
+    (torch.float32, (8, 768, 776, 1016, 1024, 1032, 4096, 5120, 8192, 12296, 16384, 16392)),
+    (torch.float16, (8, 1024, 1032, 1536, 1544, 2040, 2048, 2056, 8192, 13824, 24576, 32768, 32776))])
 def test_float_rows_bit_exact(device, dtype, widths, weight):
     rng = np.random.default_rng(5)
     for K in widths:

@@ -270,8 +270,8 @@ __global__ __launch_bounds__(kWavesPerBlock * kLanes) void k_swiglu_quant(
 // and compute in binary32, fp8_linear.py:72,77,89-90; its weight branch
 // divides in the weight's own type, fp8_linear.py:264-265), for models that
 // do not run in bf16. Quantizers: four waves per row, the row held in registers
-// (k_rowquant_float); rows past that, and SwiGLU, one wave per row and two sweeps
-// (the row maximum, then the codes, the second reading the row again).
+// (k_rowquant_float); rows past that, short ones, and SwiGLU, one wave per row and two
+// sweeps (the row maximum, then the codes, the second reading the row again).
 // ---------------------------------------------------------------------------
 
 // torch's cast to e4m3fn does not saturate: a magnitude above 464 (halfway
@@ -1321,14 +1321,19 @@ int check_typed_rows(const char* what, const void* x, int dtype, int64_t M, int6
 
 // The float row quantizers by the row's 16-byte pieces: 256 per workgroup and step, up to 16
 // steps in registers, past that (and past the rows that fit one launch of a workgroup each)
-// the two sweeps.
+// the two sweeps. Short rows go there too: four to a workgroup and no barrier, where a
+// workgroup per row leaves waves without a piece. 100000 rows, one MI355X, two sweeps against
+// one row per workgroup: binary32 64 wide 21 / 44 us, 512 44 / 68, 768 74 / 82, 832 90 / 88, 1024
+// 101 / 92; binary16 512 42 / 60, 960 74 / 76, 1024 77 / 75 (20000 rows 16.5 / 17.5), 1032 99 / 87;
+// binary16 weights 1024 75 / 89, 1536 111 / 113, 1792 139 / 125.
 template <typename T, bool kWeight>
 int launch_rowquant_float(const char* what, const T* x, int64_t M, int64_t K, int64_t ldx, uint8_t* y, int64_t ldy,
                           float* scale, hipStream_t stream)
 {
     const dim3 block(kWavesPerBlock * kLanes);
     const int64_t per = (K / FloatRow<T>::kPer + kWavesPerBlock * kLanes - 1) / (kWavesPerBlock * kLanes);
-    if (per > 16 || M >= 1 << 24) {   // (a launch takes fewer than 2^32 work-items: 2^24 workgroups)
+    const int64_t short_pieces = 64 * (sizeof(T) == 4 || kWeight ? 3 : 2);   // a wave's steps in one sweep
+    if (per > 16 || K / FloatRow<T>::kPer <= short_pieces || M >= 1 << 24) {   // (a launch takes fewer than 2^32 work-items: 2^24 workgroups)
         const dim3 grid((unsigned)((M + kWavesPerBlock - 1) / kWavesPerBlock));
         hipLaunchKernelGGL((k_rowquant_float_wide<T, kWeight>), grid, block, 0, stream, x, M, K, ldx, y, ldy, scale);
         return check_launch(what);
