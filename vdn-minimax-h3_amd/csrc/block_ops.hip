@@ -96,6 +96,13 @@ int launch_gated_residual(const uint16_t* residual, int64_t ldr, const uint16_t*
                           uint16_t* out, int64_t ldo, int64_t M, int64_t N, hipStream_t stream)
 {
     const int64_t spans = (N / 8 + kBatch * kLanes - 1) / (kBatch * kLanes);   // waves per row
+    const int64_t slab = 4 * kLaunchRows / spans > 0 ? 4 * kLaunchRows / spans : 1;   // (four waves per workgroup)
+    if (M > slab)
+        return in_slabs(M, slab, [&](int64_t m, int64_t rows) {
+            return launch_gated_residual(residual ? residual + m * ldr : nullptr, ldr, gate, ldgate,
+                                         gate_index ? gate_index + m : nullptr, gate_rows, branch + m * ldb, ldb,
+                                         out + m * ldo, ldo, rows, N, stream);
+        });
     const dim3 grid((unsigned)((M * spans + kWavesPerBlock - 1) / kWavesPerBlock)), block(kWavesPerBlock * kLanes);
     const bool nt = M * N * 2 >= kNtStoreBytes;
 #define VDN_GR(R, T)                                                                                         \

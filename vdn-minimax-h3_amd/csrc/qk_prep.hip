@@ -266,6 +266,14 @@ extern "C" int vdn_fp8_qk_prep(const void* x, int64_t T, int64_t H, int64_t d, i
     const int64_t nch = H * d / 8;
     const int cpl = pick_cpl(nch);
     if (cpl == 0) return set_error(VDN_FP8_EINVAL, "qk_prep: H * d = %lld above the supported 16384", (long long)(H * d));
+    if (T > kLaunchRows) {
+        const int64_t table = cs_bf16 ? 2 : 4;   // bytes of a table value
+        auto at = [&](const void* t, int64_t m) { return t ? (const void*)((const uint8_t*)t + m * ldcs * table) : nullptr; };
+        return in_slabs(T, kLaunchRows, [&](int64_t m, int64_t rows) {
+            return vdn_fp8_qk_prep((const uint16_t*)x + m * ldx, rows, H, d, ldx, weight, eps, at(cos, m), at(sin, m), rotary_dim, ldcs,
+                                   cs_bf16, (uint16_t*)out + m * ldo, ldo, stream);
+        });
+    }
     QkArgs p{(const uint16_t*)x, T, H, d, ldx, (const uint16_t*)weight, eps, cos, sin, rotary_dim, ldcs, cs_bf16,
              (uint16_t*)out, ldo};
     switch (d) {

@@ -1093,6 +1093,10 @@ extern "C" int vdn_fp8_quantize_rows(const void* x, int64_t M, int64_t K, int64_
                          (long long)K, (long long)ldx, (long long)ldy);
     if (!aligned(x, 16) || !aligned(y, 8) || !aligned(scale, 4))
         return set_error(VDN_FP8_EINVAL, "quantize_rows: x must be 16-byte and y 8-byte aligned");
+    if (M > kLaunchRows)
+        return in_slabs(M, kLaunchRows, [&](int64_t m, int64_t rows) {
+            return vdn_fp8_quantize_rows((const uint16_t*)x + m * ldx, rows, K, ldx, (uint8_t*)y + m * ldy, ldy, scale + m, stream);
+        });
     const dim3 grid((unsigned)((M + kWavesPerBlock - 1) / kWavesPerBlock));
     launch_rowquant<false>(pick_cpl(K / 8), grid, stream, (const uint16_t*)x, M, K, ldx, (uint8_t*)y, ldy, scale);
     return check_launch("quantize_rows");
@@ -1113,6 +1117,10 @@ extern "C" int vdn_fp8_gelu_quantize_rows(const void* h, int64_t M, int64_t K, i
     if (!aligned(h, 16) || !aligned(y, 8) || !aligned(scale, 4))
         return set_error(VDN_FP8_EINVAL, "gelu_quantize_rows: h must be 16-byte and y 8-byte aligned");
     if (K / 8 > 32 * kLanes) return set_error(VDN_FP8_EINVAL, "gelu_quantize_rows: K=%lld above the supported 16384", (long long)K);
+    if (M > kLaunchRows)
+        return in_slabs(M, kLaunchRows, [&](int64_t m, int64_t rows) {
+            return vdn_fp8_gelu_quantize_rows((const uint16_t*)h + m * ldh, rows, K, ldh, (uint8_t*)y + m * ldy, ldy, scale + m, stream);
+        });
     const dim3 grid((unsigned)((M + kWavesPerBlock - 1) / kWavesPerBlock));
     launch_rowquant<false, true>(pick_cpl(K / 8), grid, stream, (const uint16_t*)h, M, K, ldh, (uint8_t*)y, ldy, scale);
     return check_launch("gelu_quantize_rows");
@@ -1130,6 +1138,10 @@ extern "C" int vdn_fp8_swiglu_quantize_rows(const void* h, int64_t M, int64_t K,
     if (!aligned(h, 16) || !aligned(y, 8)) return set_error(VDN_FP8_EINVAL, "swiglu_quantize_rows: misaligned pointer");
     const int64_t nch = K / 8;
     if (nch > 32 * kLanes) return set_error(VDN_FP8_EINVAL, "swiglu_quantize_rows: K=%lld above the supported 16384", (long long)K);
+    if (M > kLaunchRows)
+        return in_slabs(M, kLaunchRows, [&](int64_t m, int64_t rows) {
+            return vdn_fp8_swiglu_quantize_rows((const uint16_t*)h + m * ldh, rows, K, ldh, (uint8_t*)y + m * ldy, ldy, scale + m, stream);
+        });
     const dim3 grid((unsigned)((M + kWavesPerBlock - 1) / kWavesPerBlock)), block(kWavesPerBlock * kLanes);
     const uint16_t* hp = (const uint16_t*)h;
     uint8_t* yp = (uint8_t*)y;
@@ -1287,6 +1299,12 @@ extern "C" int vdn_fp8_requantize_weight(const void* w, int64_t N, int64_t K, in
         return launch_lora_requant((const uint16_t*)w, N, K, ldw, (const uint16_t*)lora_a, (const uint16_t*)lora_b,
                                    rank, lora_scale, (uint8_t*)wq, ldq, w_scale, (uint16_t*)w_merged, stream);
     }
+    if (N > kLaunchRows)
+        return in_slabs(N, kLaunchRows, [&](int64_t n, int64_t rows) {
+            return vdn_fp8_requantize_weight((const uint16_t*)w + n * ldw, rows, K, ldw, nullptr, nullptr, 0, 0.0f,
+                                             (uint8_t*)wq + n * ldq, ldq, w_scale + n,
+                                             w_merged ? (uint16_t*)w_merged + n * ldw : nullptr, stream);
+        });
     const dim3 grid((unsigned)((N + kWavesPerBlock - 1) / kWavesPerBlock));
     launch_rowquant<true>(pick_cpl(K / 8), grid, stream, (const uint16_t*)w, N, K, ldw, (uint8_t*)wq, ldq, w_scale);
     int st = check_launch("requantize_weight");
@@ -1320,8 +1338,7 @@ int check_typed_rows(const char* what, const void* x, int dtype, int64_t M, int6
 }
 
 // The float row quantizers by the row's 16-byte pieces: 256 per workgroup and step, up to 16
-// steps in registers, past that (and past the rows that fit one launch of a workgroup each)
-// the two sweeps. Short rows go there too: four to a workgroup and no barrier, where a
+// steps in registers, past that the two sweeps. Short rows go there too: four to a workgroup and no barrier, where a
 // workgroup per row leaves waves without a piece. 100000 rows, one MI355X, two sweeps against
 // one row per workgroup: binary32 64 wide 21 / 44 us, 512 44 / 68, 768 74 / 82, 832 90 / 88, 1024
 // 101 / 92; binary16 512 42 / 60, 960 74 / 76, 1024 77 / 75 (20000 rows 16.5 / 17.5), 1032 99 / 87;
@@ -1330,10 +1347,14 @@ template <typename T, bool kWeight>
 int launch_rowquant_float(const char* what, const T* x, int64_t M, int64_t K, int64_t ldx, uint8_t* y, int64_t ldy,
                           float* scale, hipStream_t stream)
 {
+    if (M > kLaunchRows)
+        return in_slabs(M, kLaunchRows, [&](int64_t m, int64_t rows) {
+            return launch_rowquant_float<T, kWeight>(what, x + m * ldx, rows, K, ldx, y + m * ldy, ldy, scale + m, stream);
+        });
     const dim3 block(kWavesPerBlock * kLanes);
     const int64_t per = (K / FloatRow<T>::kPer + kWavesPerBlock * kLanes - 1) / (kWavesPerBlock * kLanes);
     const int64_t short_pieces = 64 * (sizeof(T) == 4 || kWeight ? 3 : 2);   // a wave's steps in one sweep
-    if (per > 16 || K / FloatRow<T>::kPer <= short_pieces || M >= 1 << 24) {   // (a launch takes fewer than 2^32 work-items: 2^24 workgroups)
+    if (per > 16 || K / FloatRow<T>::kPer <= short_pieces) {
         const dim3 grid((unsigned)((M + kWavesPerBlock - 1) / kWavesPerBlock));
         hipLaunchKernelGGL((k_rowquant_float_wide<T, kWeight>), grid, block, 0, stream, x, M, K, ldx, y, ldy, scale);
         return check_launch(what);
@@ -1366,6 +1387,11 @@ extern "C" int vdn_fp8_swiglu_quantize_rows_typed(const void* h, int dtype, int6
     if (dtype == VDN_FP8_DTYPE_BF16) return vdn_fp8_swiglu_quantize_rows(h, M, K, ldh, y, ldy, scale, stream);
     const int st = check_typed_rows("swiglu_quantize_rows", h, dtype, M, K, ldh, 2 * K, y, ldy, scale);
     if (st >= 0) return st;
+    if (M > kLaunchRows)
+        return in_slabs(M, kLaunchRows, [&](int64_t m, int64_t rows) {
+            return vdn_fp8_swiglu_quantize_rows_typed((const uint8_t*)h + m * ldh * (dtype == VDN_FP8_DTYPE_F32 ? 4 : 2), dtype, rows,
+                                                      K, ldh, (uint8_t*)y + m * ldy, ldy, scale + m, stream);
+        });
     const dim3 grid((unsigned)((M + kWavesPerBlock - 1) / kWavesPerBlock)), block(kWavesPerBlock * kLanes);
     if (dtype == VDN_FP8_DTYPE_F32)
         hipLaunchKernelGGL((k_swiglu_quant_float<float>), grid, block, 0, stream, (const float*)h, M, K, ldh,

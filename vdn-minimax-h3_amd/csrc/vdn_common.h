@@ -28,6 +28,20 @@ int device_cus();
 // nch chunks with one wave; 0 above 32 x 64 chunks.
 int pick_cpl(int64_t nch);
 
+// Rows that a row kernel's launch takes, at most a workgroup of 256 threads each: HIP takes
+// fewer than 2^32 work-items in a launch, and of more it starts only the remainder, without an
+// error. More rows go in slabs: launch(first row, rows) for each.
+constexpr int64_t kLaunchRows = 1 << 23;
+template <typename F>
+int in_slabs(int64_t rows, int64_t slab, F launch)
+{
+    for (int64_t m = 0; m < rows; m += slab) {
+        const int st = launch(m, rows - m < slab ? rows - m : slab);
+        if (st != VDN_FP8_OK) return st;
+    }
+    return VDN_FP8_OK;
+}
+
 inline bool aligned(const void* p, uintptr_t a) { return ((uintptr_t)p % a) == 0; }
 
 // ---------------------------------------------------------------------------
