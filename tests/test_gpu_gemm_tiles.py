@@ -10,6 +10,7 @@ import torch
 
 import vdn_fp8
 import vdn_fp8._lib as L
+from conftest import gemm_plan
 
 pytestmark = pytest.mark.gpu
 
@@ -100,3 +101,29 @@ def test_the_answered_workspace_is_enough(device, M, N, K, out):
     torch.cuda.synchronize()
     if ws.numel() == 16:
         assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))   # no split either way
+
+
+def test_more_tiles_than_a_launch_holds(device):
+    """2^24 workgroups of 256 threads pass what one launch starts: the rows go in halves."""
+    M, N, K = 192 * (1 << 24) + 5, 4, 16
+    need = M * (K + 4 + 2 * N)
+    if torch.cuda.mem_get_info(device)[0] < need + (16 << 30):
+        pytest.skip(f"needs {need >> 30} GiB of GPU memory")
+    print(f"gemm [{M}, {N}, {K}], plan {gemm_plan(M, N, K, False, cus=0)}", flush=True)
+    xq = torch.zeros(M, K, device=device, dtype=torch.uint8)
+    rows = [0, 1, M // 2, M // 2 + 511, 192 * (1 << 24) - 1, 192 * (1 << 24), M - 1]
+    for i, r in enumerate(rows):
+        xq[r, i] = 0x38                                        # 1.0
+    sx, sw = torch.ones(M, device=device), torch.arange(1.0, N + 1, device=device)
+    wq = torch.full((N, K), 0x38, device=device, dtype=torch.uint8)
+    out = torch.full((M, N), 7.0, device=device, dtype=torch.bfloat16)
+    st = torch.cuda.current_stream().cuda_stream
+    L.check(L.load().vdn_fp8_gemm(xq.data_ptr(), sx.data_ptr(), wq.data_ptr(), sw.data_ptr(), M, N, K, K, K, None, L.EPI_NONE,
+                                  None, None, 0, 0, None, 0, out.data_ptr(), N, st), "gemm")
+    torch.cuda.synchronize()
+    for r in rows:
+        assert torch.equal(out[r].float(), sw), r
+        out[r] = 0
+    assert not any(bool(out[i:i + (1 << 28)].any()) for i in range(0, M, 1 << 28))
+    del xq, sx, out
+    torch.cuda.empty_cache()

@@ -1017,6 +1017,25 @@ int gemm_launch(const void* xq, const float* x_scale, const void* wq, const floa
                epilogue == VDN_FP8_EPI_F32 && out_type < 0 ? VDN_FP8_DTYPE_F32 : std::max(out_type, 0), (int)tiles_m, (int)tiles_n,
                kGroupM, plan.t_main, plan.splits, plan.units, ws};
     const bool tile_fast = out16 && (!gated || rows31);
+    const int64_t part_m = plan.main ? 1 : (M + 32 * plan.b - 1) / (32 * plan.b), part_n = plan.main ? 1 : (N + 32 * plan.a - 1) / (32 * plan.a);
+    if (part_m * part_n >= 1 << 24) {
+        // A launch of 2^24 workgroups passes 2^32 work-items, of which HIP starts only the remainder:
+        // two halves, each planned by itself. (Here rather than by a second grid dimension, whose
+        // index cost the tile kernel 0.5 us of [821, 5376, 5120]'s 27.)
+        const int64_t hm = part_m >= part_n ? (M / 2 + 255) / 256 * 256 : 0, hn = hm ? 0 : (N / 2 + 255) / 256 * 256;
+        const int64_t be = p.out_type == VDN_FP8_DTYPE_F32 ? 4 : 2;   // bytes of a bias value and of an output
+        for (int h = 0; h < 2; ++h) {
+            const int64_t m0 = h ? hm : 0, n0 = h ? hn : 0;
+            auto at = [](const void* t, int64_t off) { return t ? (const void*)((const uint8_t*)t + off) : nullptr; };
+            const int st = gemm_launch(p.xq + m0 * ldx, x_scale + m0, p.wq + n0 * ldw, w_scale + n0,
+                                       hm ? (h ? M - hm : hm) : M, hn ? (h ? N - hn : hn) : N, K, ldx, ldw, at(bias, n0 * be), epilogue,
+                                       at(gate, n0 * 2), (const int32_t*)at(gate_index, m0 * 4), gate_rows, ldgate,
+                                       at(residual, (m0 * ldres + n0) * 2), ldres, (uint8_t*)out + (m0 * ldo + n0) * be, ldo, nullptr, 0,
+                                       stream, out_type);
+            if (st != VDN_FP8_OK) return st;
+        }
+        return VDN_FP8_OK;
+    }
     if (!plan.main) return launch_gemm_tile(p, plan.a, plan.b, 0, epilogue, tile_fast, stream);
     const int64_t need = (int64_t)plan.units * kUnitFloats * (int64_t)sizeof(float);
     if (ws_bytes < need)

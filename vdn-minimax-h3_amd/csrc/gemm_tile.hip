@@ -88,7 +88,9 @@ void k_gemm_tile(GemmArgs p, int epi, int fast)
 #pragma unroll
     for (int i = 0; i < A; ++i) woff[i] = (uint32_t)((8 * A * wave + 8 * i + (lane >> 3)) * p.ldw) + chunk16;
     // Copy c of block kb into stage st; blocks past the last one still issue theirs, through
-    // empty descriptors (zeros, no memory read), so that the counts the waits rely on hold.
+    // empty descriptors (zeros, no memory read), so that the counts the waits rely on hold. (The
+    // part adds the scalar offset before it compares with the range, and does not wrap: copies
+    // of a zero range at scalar offsets inside a buffer gave zeros.)
     auto copy = [&](uint32_t st, int kb, int c) {
         const bool out = kb * BK + chunk16 >= (int)p.K;   // this lane's 16 bytes lie past K
         const int live = kb < nk ? -1 : 0;
