@@ -182,3 +182,23 @@ def test_library_from_another_compiler_is_refused(tmp_path):
     env = dict(os.environ, HIPCC=str(fake))
     r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=120)
     assert "REFUSED" in r.stdout and "compiler" in r.stdout, r.stdout + r.stderr
+
+
+def test_kernel_families_hold_every_file_they_are_made_of():
+    """A family's digest covers every source named after it and every header that those include,
+    so that a profile keyed to it is not taken for one of other code."""
+    from vdn_fp8 import build as B
+    covered = set()
+    for family, files in B.KERNEL_FILES.items():
+        named = [s for s in B.SOURCES if s == family + ".hip" or s.startswith(family + "_")]
+        need, todo = set(), list(named)
+        while todo:
+            f = todo.pop()
+            if f in need:
+                continue
+            need.add(f)
+            path = os.path.join(B.INCLUDE if f in B.PUBLIC_HEADERS else B.CSRC, f)
+            todo += [h for h in re.findall(r'#include "(\w+\.h)"', open(path).read()) if h in B.HEADERS + B.PUBLIC_HEADERS]
+        assert named and need <= set(files), (family, sorted(need - set(files)))
+        covered |= set(files)
+    assert {"gemm_tile.hip", "gemm_common.h"} <= covered

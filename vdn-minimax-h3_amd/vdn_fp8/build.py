@@ -90,7 +90,7 @@ def source_manifest(csrc=CSRC, include=INCLUDE, compiler=None):
 
 # The files that make each kernel family (its source plus the shared headers).
 KERNEL_FILES = {
-    "gemm": ["gemm.hip", "gemm_common.h", "vdn_common.h", "vdn_fp8.h"],
+    "gemm": ["gemm.hip", "gemm_tile.hip", "gemm_common.h", "vdn_common.h", "vdn_fp8.h"],
     "quantize": ["quantize.hip", "vdn_common.h", "vdn_fp8.h"],
     "lora_requant": ["lora_requant.hip", "quantize.hip", "vdn_common.h", "vdn_fp8.h"],
 }
