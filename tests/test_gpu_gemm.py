@@ -20,7 +20,7 @@ import torch
 
 import oracle as O
 import vdn_fp8
-from conftest import bits, codes, from_bits
+from conftest import bits, codes, from_bits, gemm_plan
 from vdn_fp8 import workloads
 
 pytestmark = pytest.mark.gpu
@@ -302,8 +302,8 @@ def test_gemm_gate_residual(device):
 @pytest.mark.parametrize("M,N,K,epi", [(300, 260, 400, "gelu_tanh"), (300, 512, 208, "gate_rows"),
                                        (257, 264, 1040, "gate_broadcast"), (130, 516, 144, "gate_rows")])
 def test_gemm_ktail_and_narrow_epilogues(device, M, N, K, epi):
-    """The epilogues on the K % 128 != 0 kernel and on output rows that are not 16-byte
-    multiples (N % 8 != 0: the general, unstaged epilogue)."""
+    """The epilogues of the tile kernel, with a partial last K block and on output rows that are
+    not 16-byte multiples (N % 8 != 0: 8-byte pieces)."""
     print(f"gemm epilogue {epi} M={M} N={N} K={K}", flush=True)
     rng = np.random.default_rng(M + N + K)
     x, w, b = _rand(rng, (M, K), 1.0), _rand(rng, (N, K), 0.05), _rand(rng, (N,), 0.1)
@@ -344,18 +344,33 @@ def test_gemm_operands_on_other_devices(device):
         f.forward_quantized(qx, sx, epilogue="gate", gate=gate, residual=torch.zeros(M, N, dtype=torch.bfloat16))
 
 
-@pytest.mark.parametrize("M,N,K", [(4096, 4352, 128), (4352, 4096, 384), (4100, 4356, 256)])
-def test_gemm_many_tiles(device, M, N, K):
-    """More 256 x 256 tiles than compute units: each workgroup walks several tiles,
-    the copy stream running across tile boundaries (K = 128: one block per tile)."""
+def _whole_tiles(device, M, N, K, rows16, want):
+    """The whole 256-row tiles of the persistent kernel in this shape's plan."""
+    if torch.cuda.get_device_properties(device).multi_processor_count == 256:
+        p = gemm_plan(M, N, K, rows16, cus=0)
+        assert (p[1] if p[0] == 256 else 0) == want, p
+
+
+@pytest.mark.parametrize("M,N,K,whole", [(4096, 4352, 128, 0), (4352, 4096, 384, 0), (4100, 4356, 256, 256),
+                                         (6700, 4100, 512, 459), (5000, 5904, 1024, 480)])
+def test_gemm_many_tiles(device, M, N, K, whole):
+    """More 256 x 256 tiles than compute units: on the tile kernel (K no multiple of 256: several
+    rounds of its tiles), a round of whole tiles and quarters behind it, and whole tiles throughout,
+    where each workgroup walks several, the copy stream running across tile boundaries
+    (N = 4100: the general epilogue, N = 5904: the fast one)."""
     print(f"gemm M={M} N={N} K={K}", flush=True)
+    _whole_tiles(device, M, N, K, N % 8 == 0, whole)
     rng = np.random.default_rng(M + N + K)
     _check(_rand(rng, (M, K), 1.0), _rand(rng, (N, K), 0.05), _rand(rng, (N,), 0.1), device)
 
 
-def test_gemm_many_tiles_gate(device):
+@pytest.mark.parametrize("M,N,K,whole", [(4352, 4100, 256, 256), (6700, 4100, 512, 459)])
+def test_gemm_many_tiles_gate(device, M, N, K, whole):
+    """Gate table and residual on rows that are not 16-byte: the persistent kernel's general
+    epilogue (a round of whole tiles with quarters behind it, and several tiles per workgroup)."""
+    _whole_tiles(device, M, N, K, False, whole)
     rng = np.random.default_rng(12)
-    M, N, K, T = 4352, 4100, 256, 5
+    T = 5
     gate = O.bf16_encode(rng.uniform(-2, 2, (T, N)).astype(np.float32))
     gi = rng.integers(-1, T + 1, M).astype(np.int32)           # out-of-range rows clamp
     res = _rand(rng, (M, N), 1.0)
@@ -364,8 +379,8 @@ def test_gemm_many_tiles_gate(device):
 
 
 def test_gemm_gate_rows_paths(device):
-    """A per-row gate on 16-byte rows runs as the GEMM then the in-place gated residual
-    kernel; misaligned residual rows take the epilogue inside the GEMM. Both against the
+    """A per-row gate on 16-byte rows, and residual rows that are not 16-byte aligned (8-byte
+    pieces). Both against the
     oracle: per-row gate without residual (signed zeros kept), and with a residual whose
     rows start 8 bytes off a 16-byte boundary."""
     rng = np.random.default_rng(14)
@@ -559,7 +574,8 @@ def test_gemm_split_k(device, M, N, K, epi):
 @pytest.mark.parametrize("M,N,K,T,order,bias,res", [
     (13107, 5376, 14336, 5, "frames", False, True),   # H3 FF down: split-K tiles through the reduction
     (1000, 1032, 1024, 4, "random", True, True),      # partial tiles in M and N, out-of-range indices
-    (777, 2048, 8192, 3, "random", False, False),     # split, per-row gate without a residual
+    (777, 2048, 8192, 3, "random", False, False),     # long rows on small tiles, no residual
+    (300, 512, 8192, 3, "random", False, False),      # split, per-row gate without a residual
     (300, 512, 5120, 1, "frames", True, True),        # one-row table with a residual
 ])
 def test_gemm_row_gate_epilogue_matches_two_kernels(device, M, N, K, T, order, bias, res):
@@ -569,6 +585,8 @@ def test_gemm_row_gate_epilogue_matches_two_kernels(device, M, N, K, T, order, b
     fused form may not move a bit. Table indices frame-ordered (the model's) or random with
     values outside the table (clamped, as the gated residual kernel clamps)."""
     import vdn_fp8._lib as L
+    if (M, K) in ((13107, 14336), (300, 8192)):
+        assert vdn_fp8.fp8_linear.gemm_workspace_bytes(M, N, K, device) > 0
     print(f"row-gate epilogue [{M}, {N}, {K}] T={T} {order} bias={bias} residual={res}", flush=True)
     g = torch.Generator(device=device).manual_seed(M + N)
     lin = torch.nn.Linear(K, N, bias=bias, device=device, dtype=torch.bfloat16)
@@ -597,13 +615,15 @@ def test_gemm_row_gate_epilogue_matches_two_kernels(device, M, N, K, T, order, b
 
 
 @pytest.mark.parametrize("epi", [None, "gelu_tanh"])
-def test_gemm_quadrant_tiles_match_whole_tiles(device, epi):
-    """A shape of few tiles runs them as quadrants (four workgroups per 256 x 256 tile, each
-    wave 64 x 64 of it); the same rows and columns inside a shape that fills a whole round
-    of the persistent kernel come out bit for bit the same: every output is the same chain
-    of MFMAs over the same K blocks, in its tile's rotated order, then the same epilogue."""
-    M, K, N, N2 = 1000, 2048, 520, 16384    # 4 x 3 tiles (quadrants); 4 x 64 = 256 tiles (whole tiles)
-    print(f"quadrant tiles [{M}, {N}, {K}] against [{M}, {N2}, {K}], epilogue {epi}", flush=True)
+def test_gemm_small_tiles_match_whole_tiles(device, epi):
+    """A shape of few 256 x 256 tiles runs on the tile kernel (72 tiles of 128 x 64 here); the
+    same rows and columns inside a shape that fills a whole round of the persistent kernel come
+    out bit for bit the same: every output is the same chain of MFMAs over the same K blocks in
+    ascending order, then the same epilogue."""
+    M, K, N, N2 = 1000, 2048, 520, 16384    # 4 x 3 tiles; 4 x 64 = 256 tiles (whole tiles)
+    _whole_tiles(device, M, N, K, True, 0)
+    _whole_tiles(device, M, N2, K, True, 256)
+    print(f"small tiles [{M}, {N}, {K}] against [{M}, {N2}, {K}], epilogue {epi}", flush=True)
     g = torch.Generator(device=device).manual_seed(41)
     lin = torch.nn.Linear(K, N2, bias=True, device=device, dtype=torch.bfloat16)
     with torch.no_grad():

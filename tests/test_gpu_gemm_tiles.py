@@ -2,9 +2,11 @@
 
 Every output is one chain of MFMAs over the 128-byte K blocks in ascending order followed by
 the same roundings, so it may not depend on the tile it falls in, on the K rows' padding
-with zero codes, or on the epilogue's store path. The problem is run as it is (the plan
-picks the tile kernel, 224-row tiles or a last round in parts) and inside one of exactly two
-rounds of whole 256 x 256 tiles of the persistent kernel, its rows, columns and K padded."""
+with zero codes, or on the epilogue's store path. The problem is run as it is (by the
+plan that its row names: the tile kernel, 224-row tiles, a last round in parts, or whole tiles
+through the general epilogue) and inside one of exactly two rounds of whole 256 x 256 tiles of
+the persistent kernel through the fast epilogue (the only one of a typed output is the general
+one), its rows, columns and K padded."""
 import pytest
 import torch
 
@@ -15,15 +17,22 @@ from conftest import gemm_plan
 pytestmark = pytest.mark.gpu
 
 MB, NB = 4096, 8192          # 16 x 32 tiles: two rounds on 256 compute units
+_TYPED = {"f16": (torch.float16, L.DTYPE_F16), "f32": (torch.float32, L.DTYPE_F32)}
 
 
 def _gemm(xq, sx, wq, sw, bias, epi, gate, gi, res, n):
+    """vdn_fp8_gemm, or with epi "f16" / "f32" vdn_fp8_gemm_typed of that output and bias."""
     M, K = xq.shape
-    out = torch.empty(M, n, device=xq.device, dtype=torch.float32 if epi == L.EPI_F32 else torch.bfloat16)
     ptr = lambda t: None if t is None else t.data_ptr()
-    L.check(L.load().vdn_fp8_gemm(ptr(xq), ptr(sx), ptr(wq), ptr(sw), M, n, K, K, K, ptr(bias), epi, ptr(gate), ptr(gi),
-                                  0 if gate is None else gate.shape[0], 0 if gate is None else n, ptr(res),
-                                  0 if res is None else n, ptr(out), n, torch.cuda.current_stream().cuda_stream), "gemm")
+    a, st = (ptr(xq), ptr(sx), ptr(wq), ptr(sw), M, n, K, K, K, ptr(bias)), torch.cuda.current_stream().cuda_stream
+    if epi in _TYPED:
+        dtype, code = _TYPED[epi]
+        out = torch.empty(M, n, device=xq.device, dtype=dtype)
+        L.check(L.load().vdn_fp8_gemm_typed(*a, code, ptr(out), n, None, 0, st), "gemm")
+        return out
+    out = torch.empty(M, n, device=xq.device, dtype=torch.bfloat16)
+    L.check(L.load().vdn_fp8_gemm(*a, epi, ptr(gate), ptr(gi), 0 if gate is None else gate.shape[0],
+                                  0 if gate is None else n, ptr(res), 0 if res is None else n, ptr(out), n, st), "gemm")
     return out
 
 
@@ -33,42 +42,67 @@ def _pad(t, *shape):
     return out
 
 
-@pytest.mark.parametrize("M,N,K,epi", [
-    (1, 260, 16, "none"),             # the smallest: one token, one partial K block
-    (65, 1032, 400, "gelu"),          # 128 x 64 tiles, K past the last whole block
-    (333, 516, 2048, "rows"),         # rows that are not 16-byte multiples: 8-byte pieces
-    (2514, 516, 256, "bias"),         # 128 x 96
-    (486, 4100, 272, "f32"),          # 128 x 128
-    (866, 4104, 1040, "rows"),        # 128 x 192, table rows and residual
-    (643, 4104, 256, "gelu"),         # 192 x 96
-    (962, 4096, 256, "gate"),         # 192 x 128, one gate row
-    (1026, 5376, 256, "rows"),        # 256 x 128
-    (1026, 5376, 656, "bias"),
-    (2317, 5376, 256, "gelu"),        # 224-row tiles of the persistent kernel
-    (2317, 5376, 512, "rows"),
-    (1928, 4096, 512, "bias"),        # 128 tiles as halves
-    (4000, 4168, 2048, "rows"),       # one round and a last one in eighths, columns past N
-    (4000, 4704, 2048, "rows"),       # one round and a last one in quarters
+# plan: rows of the persistent kernel's tiles, tiles it runs whole, channels and tokens of the
+# tile kernel's (on 256 compute units)
+@pytest.mark.parametrize("M,N,K,epi,plan", [
+    (1, 260, 16, "none", (0, 0, 128, 64)),             # the smallest: one token, one partial K block
+    (65, 1032, 400, "gelu", (0, 0, 128, 64)),          # K past the last whole block
+    (333, 516, 2048, "rows", (0, 0, 128, 64)),         # rows that are not 16-byte multiples: 8-byte pieces
+    (2514, 516, 256, "bias", (0, 0, 128, 64)),
+    (486, 4100, 272, "f32", (0, 0, 128, 96)),
+    (643, 4104, 256, "gelu", (0, 0, 128, 96)),
+    (2938, 800, 656, "rows", (0, 0, 128, 96)),
+    (866, 4104, 1040, "rows", (0, 0, 128, 128)),       # table rows and residual
+    (1481, 2580, 656, "f16", (0, 0, 128, 128)),        # a binary16 output with its bias
+    (962, 4096, 256, "gate", (256, 0, 128, 128)),      # 64 tiles as quarters, one gate row
+    (1026, 5376, 256, "rows", (0, 0, 128, 192)),
+    (1026, 5376, 656, "bias", (0, 0, 128, 192)),
+    (2021, 2124, 1296, "gate", (0, 0, 128, 192)),
+    (649, 6400, 768, "rows", (0, 0, 192, 96)),
+    (3431, 2476, 400, "gelu", (0, 0, 192, 96)),
+    (3078, 1856, 656, "f16", (0, 0, 192, 128)),        # 16-byte binary16 rows
+    (1772, 2524, 768, "rows", (0, 0, 192, 128)),
+    (2951, 5376, 400, "rows", (0, 0, 256, 128)),
+    (3437, 4580, 400, "f32", (0, 0, 256, 128)),
+    (2317, 5376, 256, "gelu", (224, 231, 0, 0)),       # 224-row tiles of the persistent kernel
+    (2317, 5376, 512, "rows", (224, 231, 0, 0)),
+    (1928, 4096, 512, "bias", (256, 0, 256, 128)),     # 128 tiles as halves
+    (2576, 7552, 2048, "rows", (256, 256, 256, 128)),  # a round, then halves
+    (3697, 6012, 768, "f16", (256, 256, 256, 128)),
+    (3392, 5192, 768, "gelu", (256, 256, 128, 128)),   # a round, then quarters
+    (2619, 6724, 256, "f32", (256, 256, 128, 128)),
+    (4000, 4704, 2048, "rows", (256, 256, 128, 128)),
+    (4000, 4168, 2048, "rows", (256, 256, 128, 64)),   # a round, then eighths: rows and columns past the end
+    (2128, 7456, 256, "gate", (256, 256, 128, 64)),
+    (2836, 5644, 256, "f16", (256, 256, 128, 64)),
+    (4000, 7420, 512, "none", (256, 464, 0, 0)),       # whole tiles through the general epilogue, in more
+    (4000, 7420, 512, "gelu", (256, 464, 0, 0)),       # than one round
+    (4000, 7420, 512, "gate", (256, 464, 0, 0)),
+    (4000, 7420, 512, "rows", (256, 464, 0, 0)),
+    (4000, 7420, 512, "f16", (256, 464, 0, 0)),
+    (4000, 7424, 512, "f32", (256, 464, 0, 0)),
 ])
-def test_tile_shapes_give_the_same_bits(device, M, N, K, epi):
+def test_tile_shapes_give_the_same_bits(device, M, N, K, epi, plan):
     print(f"gemm tiles [{M}, {N}, {K}] {epi}", flush=True)
+    KB = -(-K // 256) * 256
+    if torch.cuda.get_device_properties(device).multi_processor_count == 256:
+        p = gemm_plan(M, N, K, N % 8 == 0 and epi not in _TYPED, cus=0)
+        assert p[:2] + p[4:] == plan and p[2:4] == (0, 0)
+        assert gemm_plan(MB, NB, KB, epi not in _TYPED, cus=0) == (256, 512, 0, 0, 0, 0)
     g = torch.Generator(device=device).manual_seed(M + N + K)
     rand = lambda *s: torch.randn(*s, device=device, generator=g)
     xq, sx = vdn_fp8.quantize_rows(_pad(rand(M, K).to(torch.bfloat16), M, K))
     wq, sw = vdn_fp8.requantize_weight((0.02 * rand(N, K)).to(torch.bfloat16))
     sx = sx.reshape(-1)
-    bias = (0.1 * rand(N)).to(torch.bfloat16) if epi != "f32" else None
+    bias = None if epi == "none" else (0.1 * rand(N)).to(_TYPED[epi][0] if epi in _TYPED else torch.bfloat16)
     gate = gi = res = None
-    code = {"none": L.EPI_NONE, "bias": L.EPI_NONE, "gelu": L.EPI_GELU_TANH, "f32": L.EPI_F32}.get(epi, L.EPI_GATE)
-    if epi == "none":
-        bias = None
+    code = epi if epi in _TYPED else {"none": L.EPI_NONE, "bias": L.EPI_NONE, "gelu": L.EPI_GELU_TANH}.get(epi, L.EPI_GATE)
     if epi == "gate":
         gate = rand(1, N).to(torch.bfloat16)
     if epi == "rows":
         gate, res = rand(3, N).to(torch.bfloat16), rand(M, N).to(torch.bfloat16)
         gi = torch.randint(-1, 4, (M,), device=device, generator=g, dtype=torch.int32)   # clamped into the table
     got = _gemm(xq, sx, wq, sw, bias, code, gate, gi, res, N)
-    KB = -(-K // 256) * 256
     u8 = lambda t, *s: _pad(t.view(torch.uint8), *s).view(torch.float8_e4m3fn)
     want = _gemm(u8(xq, MB, KB), _pad(sx, MB), u8(wq, NB, KB), _pad(sw, NB), None if bias is None else _pad(bias, NB),
                  code, None if gate is None else _pad(gate, gate.shape[0], NB), None if gi is None else _pad(gi, MB),
