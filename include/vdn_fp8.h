@@ -185,10 +185,10 @@ int vdn_fp8_requantize_weight_typed(const void *w, int dtype, int64_t N, int64_t
  * bias bf16 [N] or NULL. For VDN_FP8_EPI_GATE: gate bf16 [gate_rows, N] (row
  * stride ldgate), gate_index int32 [M] (NULL = row 0 for every m; an index
  * outside [0, gate_rows) is clamped into it), residual bf16 [M, N] (row stride
- * ldres) or NULL. out bf16 [M, N] (row stride ldo). A per-row gate or a
- * residual on 16-byte aligned rows applies in the GEMM's epilogue; on other
- * rows, or rows whose byte offsets within 256 rows exceed 31 bits, the call
- * runs two kernels on the stream (the GEMM writing v, then the gated residual
+ * ldres) or NULL. out bf16 [M, N] (row stride ldo). The gate and the residual
+ * apply in the GEMM's epilogue; where rows are 16-byte aligned and their byte
+ * offsets within 256 rows (or the table's) exceed 31 bits, the call may run two
+ * kernels on the stream instead (the GEMM writing v, then the gated residual
  * add in place on out). The result is the same.
  * Replaces: Fp8Linear.forward_quantized, src/models/ops/fp8_linear.py:270-277
  *           (torch._scaled_mm rowwise + bias add); the GELU epilogue has no
@@ -196,9 +196,8 @@ int vdn_fp8_requantize_weight_typed(const void *w, int dtype, int64_t N, int64_t
  *           the compiled `post`, src/models/ops/fused_block.py:47-49,101-110.
  * VDN_FP8_EPI_F32 writes the binary32 x_scale[m] * w_scale[n] * acc[m][n] to
  * out (float [M, N], row stride ldo in floats, 16-byte aligned) with bias, gate
- * and residual NULL: the reference's _scaled_mm with out_dtype binary32 (the
- * caller rounds to binary16 and adds the bias for the other types, as the
- * reference does).
+ * and residual NULL: the reference's _scaled_mm with out_dtype binary32 (a
+ * binary16 output or a bias: vdn_fp8_gemm_typed).
  * Requires: K % 16 == 0; ldx, ldw % 16 == 0; ldo, ldres, ldgate % 4 == 0;
  *           xq, wq, x_scale, w_scale, bias, gate_index 16-byte aligned;
  *           out, residual, gate 8-byte aligned.
@@ -241,10 +240,13 @@ int vdn_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, int rows16, int workspace
 /*
  * vdn_fp8_gemm with a caller-provided split-K workspace (device memory, 16-byte
  * aligned, at least vdn_fp8_gemm_workspace_size bytes; NULL: no split, the same
- * call as vdn_fp8_gemm). The summation order of an output depends only on K and
- * the split, so a shape gives the same bits call after call, alone or as part of
- * a larger one; a split shape's last-round tiles sum their K slices in binary32 after
- * the matrix cores, so their bits can differ from vdn_fp8_gemm's by a rounding.
+ * call as vdn_fp8_gemm). A shape gives the same bits call after call. Without a
+ * split (K < 8192, no workspace, or a size query of 0) the summation order of an
+ * output depends only on K, so its rows and columns also have the bits they have as
+ * part of a larger shape. In a shape that splits, the tiles of the last round sum
+ * their K slices in binary32 after the matrix cores: which outputs those are, and
+ * the number of slices, depend on M, N and K, and their bits can differ from
+ * vdn_fp8_gemm's by a rounding.
  * Replaces: Fp8Linear.forward_quantized, src/models/ops/fp8_linear.py:270-277,
  *           as vdn_fp8_gemm does.
  * Requires: as vdn_fp8_gemm; workspace_bytes >= the size query's answer.

@@ -902,7 +902,11 @@ GemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int cus, bool split_ok, bool
                 if (split_ok && K >= kSplitMinK && S >= 2) {
                     const double split_us = base + nk / (double)S * 1.2 + 14.0 + 0.07 * (double)(R * S);
                     const GemmPlan split{true, 8, (int)(T - R), (int)S, (int)(R * S), 0, 0};
-                    // (at most 16 tiles over such rows: callers hold workspaces for them)
+                    // At most 16 tiles always split, so that the size query's answer for such an output
+                    // stays what it has been. On one MI355X, split against whole chains of small
+                    // tiles (what a call without a workspace runs): [256, 4096, 28672] 52 / 101 us,
+                    // [1024, 1024, 32768] 48 / 62, [300, 512, 14336] 30 / 32, [1024, 1024, 14336] 36 / 33, but
+                    // [1000, 1024, 8192] 31 / 19 and [300, 512, 8192] 25 / 19.
                     if (T <= 16) {
                         if (est) *est = split_us;
                         return split;

@@ -19,8 +19,8 @@ implemented; the per-tensor family (quantize_tensor & co.) is not part of this m
 
 Float types: as the reference, the quantizers take bf16, float16 or float32 rows (computed
 in binary32), Fp8Linear takes a Linear of any of the three (the weight's quotient in its own
-type), and `forward` returns the rows' type (vdn_fp8_*_typed and the GEMM's binary32
-output; the float16 cast and the bias add then follow as the reference's own ops).
+type), and `forward` returns the rows' type (vdn_fp8_*_typed: the cast and a bias of that type
+in the GEMM's epilogue, rounded as the reference's own ops; any other bias as its own add).
 
 Extensions (keyword-only, additive): `Fp8Linear.forward_quantized` and `forward` take an
 `epilogue` ("gelu_tanh" or "gate") with `gate`, `gate_index` and `residual`, fused into
@@ -382,11 +382,13 @@ class Fp8Linear(nn.Module):
 
         Computes bf16(epi(x_scale * w_scale * (x_fp8 @ weight_fp8.T) + bias)) in one
         kernel; with out_dtype float32 or float16 (a model that does not run in bf16: what
-        `forward` passes for such rows, as the reference does) the GEMM writes the binary32
-        product, then the cast and `+ bias` follow as in the reference. epilogue: None, "gelu_tanh", or "gate" -- gate [T, N] (or [N]) table,
-        gate_index [M] rows of it (None = row 0; out-of-range indices are clamped),
-        residual [M, N] (optional): gate[gate_index] * out + residual, the gated residual
-        add of the block (fused_block.py:47-49)."""
+        `forward` passes for such rows, as the reference does) its epilogue rounds the binary32
+        product to that type and adds a bias Parameter of it, as the reference's two ops round;
+        a bias that promotes, takes a gradient or is no plain Parameter is added after it.
+        epilogue: None, "gelu_tanh", or "gate" -- gate [T, N] (or [N]) table, gate_index [M] rows
+        of it (None = row 0; out-of-range indices are clamped), residual [M, N] (optional):
+        gate[gate_index] * out + residual, the gated residual add of the block
+        (fused_block.py:47-49)."""
         if out_dtype not in _DTYPES:
             raise ValueError(f"the fp8 GEMM writes bfloat16, float16 or float32 (out_dtype={out_dtype})")
         if out_dtype != torch.bfloat16 and (epilogue is not None or gate is not None or residual is not None):
