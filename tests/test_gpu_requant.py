@@ -201,11 +201,12 @@ def test_merge_only_in_place(device):
 
 
 @pytest.mark.parametrize("N,K,r", [(1, 5376, 8), (33, 5376, 64), (257, 5376, 32), (40, 5136, 64), (9, 5360, 16),
-                                   (5, 5392, 64)])
+                                   (5, 5392, 64), (2304, 5376, 64), (2305, 5376, 64), (2400, 5136, 32), (2311, 5360, 16),
+                                   (8203, 5376, 8)])
 @pytest.mark.parametrize("merged", [False, True])
 def test_requant_lora_21_chunks(device, N, K, r, merged):
-    """Rows of 5121 to 5376 elements, whose 21st chunk of 256 columns is a part of its own (K =
-    5392: past it, two passes). Codes and scales bit-exact with the oracle: the factors are
+    """Rows of 5121 to 5376 elements, whose 21st chunk of 256 columns is a part of its own (more
+    than 2304 rows on 256 compute units; fewer, and K = 5392, take two passes). Codes and scales bit-exact with the oracle: the factors are
     small integers over powers of two, so the update is exact in any order."""
     print(f"lora requant, 21 chunks: N={N} K={K} r={r} merged={merged}", flush=True)
     rng = np.random.default_rng(N + K + r)

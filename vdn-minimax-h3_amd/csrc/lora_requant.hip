@@ -8,7 +8,8 @@
 // quantizes it in eager torch (fp8_linear.py:262-267): several full passes over
 // W plus the write-back of W'. Here W' is never stored unless asked for.
 //
-// Two kernels. k_lora_rows (further down; rank <= 64, K <= 5376, 16-byte rows)
+// Two kernels. k_lora_rows (further down; rank <= 64, K <= 5376, 16-byte rows; past 5120
+// columns more than 2304 rows)
 // reads W once: a workgroup holds a group of whole rows of W' in registers
 // until their maximum is known, then writes the codes. k_lora_stripes (first)
 // serves everything else -- ranks up to 128, longer rows, unaligned operands,
@@ -999,7 +1000,12 @@ int launch_lora_requant(const uint16_t* w, int64_t N, int64_t K, int64_t ldw, co
     // 256 at rank <= 32, one spilled at rank 64, five with the merged rows written too. H3's
     // 5376 columns against the two passes, W from HBM: [7168, 5376] rank 64 50.1 -> 27.6 us,
     // [28672, 5376] 166 -> 108 us, rank 16 157 -> 90 us, with the merged weight 273 -> 178 us.)
+    // Past 5120 columns only for more than nine rows per compute unit: fewer are bound by one
+    // group's chain of chunks, which the two passes spread over stripes. K = 5376, two passes
+    // against one: rank 32 N = 64 17.4 / 19.9 us, 1024 17.3 / 20.2, 2304 20.0 / 20.4, 2432 23.2 /
+    // 20.6; rank 64 N = 64 17.4 / 21.4, 2304 23.2 / 23.5, 2432 27.4 / 23.7.
     const bool one_pass = !merge_only && rank <= 64 && b_vec && K <= (int64_t)rows::kChunk * rows::kMaxChunks &&
+                          (K <= (int64_t)rows::kChunk * 20 || N > 9 * (int64_t)cus) &&
                           aligned(w, 16) && ldw % 8 == 0 && aligned(wq, 16) && ldq % 16 == 0 &&
                           (!w_merged || aligned(w_merged, 16)) && (int64_t)rows::kRows * ldw * 2 <= 0x7fffffffLL &&
                           (int64_t)rows::kRows * ldq <= 0x7fffffffLL && rank * K * 2 <= 0x7fffffffLL;
